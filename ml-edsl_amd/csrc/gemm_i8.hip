@@ -7,21 +7,29 @@
 // 301-339). ReLU on i32 is tensor_map(v -> If(v > 0, v, 0))
 // (LinalgBuilder.cpp:141-178).
 //
-// Fast path (int8 matrix cores): when every X and W value lies in [-128, 127]
-// the product can run on v_mfma_i32_32x32x32_i8 exactly: each product fits in
+// Every product runs on the int8 matrix cores (v_mfma_i32_32x32x32_i8),
+// exactly. When every X and W value lies in [-128, 127] each product fits in
 // 15 bits and the i32 accumulator cannot overflow for K < 2^17, so the sum
 // equals the exact integer sum -- identical to the wrapping i32 sum in any
-// order. A pre-pass narrows X and W to int8 and writes them fragment-packed
-// (each 32x32 block stored as the 64 lanes x 16 bytes the MFMA consumes, W
-// transposed on the way), and flags any out-of-range value. The packed copies
-// are padded with zeros to multiples of the 128-wide tile in M, N and K, so
-// any shape runs on the matrix cores; the GEMM stores only the real M x N.
-// The pre-pass writes one range flag per 64x64 tile of X and of W on every
-// call (1: some value outside int8, else 0). Each GEMM workgroup reads the
-// flags of the X row panels and W column panels its tile uses; if any is set,
-// that tile alone takes the exact wrapping-i32 vector-ALU path on the
-// original i32 tensors instead. Every flag is rewritten by every call, so a
-// replayed graph never sees a previous call's state.
+// order. Wider values are written in signed base-256 digits, v = sum_d 256^d
+// v_d modulo 2^32 (at most four), and the product modulo 2^32 is the sum of
+// the digit products X_i W_j with i + j <= 3, each such an int8 product,
+// shifted by 8 (i + j). Only the pairs that the values need are run: a layer
+// whose X holds 16-bit activations and whose W is int8 costs two int8 products
+// (512x1024x512: 12.9 us, 28.5 us with full 32-bit values on both sides; the
+// wrapping i32 product on the vector ALUs that this replaced: 405 us; 2048^3:
+// 40.6 and 133 us against 1169 us).
+//
+// A pre-pass narrows X and W and writes them fragment-packed, one plane a
+// digit (each 32x32 block stored as the 64 lanes x 16 bytes the MFMA consumes,
+// W transposed on the way). The packed copies are padded with zeros to
+// multiples of the 128-wide tile in M, N and K, so any shape runs on the
+// matrix cores; the GEMM stores only the real M x N. The pre-pass writes one
+// digit count per 64x64 tile of X and of W on every call, so a replayed graph
+// never sees a previous call's state. A GEMM workgroup reads the counts of the
+// X row panels and W column panels its tile uses and, where all are 1, runs
+// the single product of the first planes. K >= 2^17 takes the wrapping i32
+// kernel on the vector ALUs.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -31,7 +39,7 @@ namespace edsl {
 namespace {
 
 // ------------------------------------------------------------------ pre-pass
-// Only used on the int8 path. The i32 sources may have any alignment / row
+// Only for K < 2^17. The i32 sources may have any alignment / row
 // stride: `vec_ok` selects 16-byte source loads.
 constexpr int kNarrowTile = 64;
 
@@ -64,6 +72,12 @@ __device__ __forceinline__ int tile_packed_offset(int r, int k) {
 // The packed tile then leaves with one 16-byte store per thread (four 1 KB
 // fragments). Tiles that reach past the real M, N or K load element by element
 // and write zeros there.
+// A tile of int8 values writes plane 0 and is done (count 1). Otherwise the
+// values still in registers are reduced digit by digit, v <- (v - d) / 256
+// with d the low byte as a signed digit, one plane a round, until every
+// remainder is a signed byte; the fourth digit is taken modulo 256, which is
+// all that arithmetic modulo 2^32 needs. Planes past a tile's count are not
+// written.
 __global__ void __launch_bounds__(256) narrow_i8_kernel(NarrowI8Args a, int vec_ok_x, int vec_ok_w) {
   __shared__ uint32_t pk[kNarrowTile * kNarrowTile / 4];
   const int tid = threadIdx.x;
@@ -71,9 +85,9 @@ __global__ void __launch_bounds__(256) narrow_i8_kernel(NarrowI8Args a, int vec_
   const int bj = 4 * (tid & 15);  // 4-column block along the source's columns
   const int x_tiles_k = a.Kp / kNarrowTile;
   const int x_tiles = (a.Mp / kNarrowTile) * x_tiles_k;
-  bool bad = false;
   int r0, k0;  // tile origin in the packed matrix's (row, k) coordinates
   int8_t* dst;
+  int64_t plane;  // bytes from one digit plane to the next
   // 4 consecutive elements of row `row` from column `col` of a source with
   // `rows` x `cols` elements; zeros past either edge.
   auto load_edge = [](const int32_t* src, int64_t ld, int rows, int cols, int row, int col) {
@@ -85,11 +99,13 @@ __global__ void __launch_bounds__(256) narrow_i8_kernel(NarrowI8Args a, int vec_
     }
     return v;
   };
-  if ((int)blockIdx.x < x_tiles) {
+  const bool is_x = (int)blockIdx.x < x_tiles;  // uniform per workgroup
+  i32x4 v[4];
+  if (is_x) {
     r0 = (blockIdx.x / x_tiles_k) * kNarrowTile;
     k0 = (blockIdx.x % x_tiles_k) * kNarrowTile;
     dst = a.X8p;
-    i32x4 v[4];
+    plane = (int64_t)a.Mp * a.Kp;
     if (r0 + kNarrowTile <= a.M && k0 + kNarrowTile <= a.K) {  // uniform per workgroup
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] = load4(a.X + (int64_t)(r0 + 4 * bi + i) * a.ldx + k0 + bj, vec_ok_x);
@@ -97,15 +113,13 @@ __global__ void __launch_bounds__(256) narrow_i8_kernel(NarrowI8Args a, int vec_
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] = load_edge(a.X, a.ldx, a.M, a.K, r0 + 4 * bi + i, k0 + bj);
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) pk[tile_packed_offset(4 * bi + i, bj) >> 2] = pack_i8x4(v[i], bad);
   } else {
     const int b = blockIdx.x - x_tiles;
     const int w_tiles_n = a.Np / kNarrowTile;
     k0 = (b / w_tiles_n) * kNarrowTile;
     r0 = (b % w_tiles_n) * kNarrowTile;  // packed rows are W's columns
     dst = a.W8p;
-    i32x4 v[4];
+    plane = (int64_t)a.Np * a.Kp;
     if (k0 + kNarrowTile <= a.K && r0 + kNarrowTile <= a.N) {  // uniform per workgroup
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] = load4(a.W + (int64_t)(k0 + 4 * bi + i) * a.ldw + r0 + bj, vec_ok_w);
@@ -113,43 +127,240 @@ __global__ void __launch_bounds__(256) narrow_i8_kernel(NarrowI8Args a, int vec_
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] = load_edge(a.W, a.ldw, a.K, a.N, k0 + 4 * bi + i, r0 + bj);
     }
-    uint32_t q[4];  // q[i] = W row k0 + 4bi + i, columns r0 + bj .. + 3 (byte e = column e)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) q[i] = pack_i8x4(v[i], bad);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      // column r0 + bj + e, rows k0 + 4bi .. + 3 as one word (byte i = row i)
-      uint32_t w = 0;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) w |= ((q[i] >> (8 * e)) & 0xffu) << (8 * i);
-      pk[tile_packed_offset(bj + e, 4 * bi) >> 2] = w;
-    }
   }
-  const int tile_bad = __syncthreads_or(bad ? 1 : 0);
   const int frag = tid >> 6, lane = tid & 63;
   const int rb = (r0 >> 5) + (frag >> 1), kt = (k0 >> 5) + (frag & 1);
-  const i32x4 out = reinterpret_cast<const i32x4*>(pk)[tid];
-  *reinterpret_cast<i32x4*>(dst + ((((int64_t)rb * (a.Kp >> 5) + kt) * 64 + lane) << 4)) = out;
+  int8_t* out = dst + ((((int64_t)rb * (a.Kp >> 5) + kt) * 64 + lane) << 4);
+  int digits = 1;
+  for (;; ++digits) {
+    bool bad = false;
+    if (is_x) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pk[tile_packed_offset(4 * bi + i, bj) >> 2] = pack_i8x4(v[i], bad);
+    } else {
+      uint32_t q[4];  // q[i] = W row k0 + 4bi + i, columns r0 + bj .. + 3 (byte e = column e)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) q[i] = pack_i8x4(v[i], bad);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        // column r0 + bj + e, rows k0 + 4bi .. + 3 as one word (byte i = row i)
+        uint32_t w = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w |= ((q[i] >> (8 * e)) & 0xffu) << (8 * i);
+        pk[tile_packed_offset(bj + e, 4 * bi) >> 2] = w;
+      }
+    }
+    const int more = __syncthreads_or(bad ? 1 : 0);
+    *reinterpret_cast<i32x4*>(out) = reinterpret_cast<const i32x4*>(pk)[tid];
+    if (!more || digits == kI8Digits) break;  // uniform
+    out += plane;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[i][e] = (int32_t)((uint32_t)v[i][e] - (uint32_t)(int32_t)(int8_t)v[i][e]) >> 8;
+    __syncthreads();  // every thread has read pk
+  }
   if (tid == 0) {
-    // Written on every call: X flags [Mp/64][Kp/64], W flags [Np/64][Kp/64].
-    uint8_t* f = dst == a.X8p ? a.flags_x : a.flags_w;
-    f[(int64_t)(r0 / kNarrowTile) * (a.Kp / kNarrowTile) + k0 / kNarrowTile] = tile_bad ? 1 : 0;
+    // Written on every call: X counts [Mp/64][Kp/64], W counts [Np/64][Kp/64].
+    uint8_t* f = is_x ? a.flags_x : a.flags_w;
+    f[(int64_t)(r0 / kNarrowTile) * (a.Kp / kNarrowTile) + k0 / kNarrowTile] = (uint8_t)digits;
   }
 }
 
-// Whether the tile at (m0, n0) must take the exact i32 path: any range flag
-// of its two 64-row X panels or its two 64-column W panels is set. Uniform
-// over the workgroup (NT threads). Flag rows of one panel are Kp/64 bytes,
-// an even count, and the two panels of a 128-wide tile are adjacent, so the
-// 2*Kp/64 flags are read as 4-byte words.
+// Whether the 128x128 tile at (m0, n0) needs more than one digit: any count
+// of its two 64-row X panels or its two 64-column W panels is above 1.
+// Uniform over the workgroup (NT threads). Count rows of one panel are Kp/64
+// bytes, an even number, and the two panels of a 128-wide tile are adjacent,
+// so the 2*Kp/64 counts are read as 4-byte words (two panels of two counts
+// each at most).
 template <int NT>
-__device__ __forceinline__ bool tile_out_of_range(const GemmI32Args& a, int m0, int n0) {
+__device__ __forceinline__ bool tile_is_wide(const GemmI32Args& a, int m0, int n0) {
   const int kt = a.Kp / kNarrowTile;
   const uint32_t* fx = reinterpret_cast<const uint32_t*>(a.flags_x + (int64_t)(m0 / kNarrowTile) * kt);
   const uint32_t* fw = reinterpret_cast<const uint32_t*>(a.flags_w + (int64_t)(n0 / kNarrowTile) * kt);
-  int bad = 0;
-  for (int i = threadIdx.x; i < kt / 2; i += NT) bad |= (fx[i] | fw[i]) != 0;
-  return __syncthreads_or(bad) != 0;
+  int wide = 0;
+  for (int i = threadIdx.x; i < kt / 2; i += NT) wide |= ((fx[i] | fw[i]) & ~0x01010101u) != 0;
+  return __syncthreads_or(wide) != 0;
+}
+
+// ------------------------------------------------------- digit-plane products
+// One wave's 64x64 outputs (2x2 blocks of 32x32) of the packed operands, over
+// the 64-k chunks first, first + stride, ...: with X = sum_i 256^i X_i and W =
+// sum_j 256^j W_j in signed base-256 digits,
+//   X W mod 2^32 = sum over i + j <= 3 of 256^(i+j) X_i W_j,
+// each X_i W_j an exact int8 product (|sum| <= 2^14 K < 2^31). The pairs are
+// taken by falling i + j, the running total shifted up by 8 between them
+// (Horner), so one accumulator and one total suffice; adds wrap as arith.addi
+// does. Counts hold one byte per 64x64 tile: the wave runs the pairs that
+// any of its chunks needs, and reads a plane that a chunk does not have (never
+// written) as zeros through an out-of-range buffer offset, as it does chunks
+// past the last. Lane l of a counts register holds the count of the wave's
+// chunk 64 * (t / 64) + l, read back by lane number.
+constexpr int kOutOfRange = 0x7fffffff;
+
+template <int D>
+__device__ __forceinline__ void digits_wave(const GemmI32Args& a, int m0, int n0, int first, int stride,
+                                            i32x16 (&total)[2][2]) {
+  const int lane = threadIdx.x & 63;
+  const int chunks = a.Kp / 64;
+  const int n = (chunks - first + stride - 1) / stride;  // this wave's chunks
+  const int block_bytes = (a.Kp >> 5) * 1024;            // one 32-row block of a plane
+  const uint8_t* fx = a.flags_x + (int64_t)(m0 / 64) * chunks + first;
+  const uint8_t* fw = a.flags_w + (int64_t)(n0 / 64) * chunks + first;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) total[i][j][r] = 0;
+  if (n <= 0) return;  // fewer chunks than waves
+  int dx = 1, dw = 1;
+  for (int t = lane; t < n; t += 64) {
+    dx = max(dx, (int)fx[(int64_t)t * stride]);
+    dw = max(dw, (int)fw[(int64_t)t * stride]);
+  }
+#pragma unroll
+  for (int d = 2; d <= kI8Digits; ++d) {  // wave maxima, uniform
+    if (__any(dx >= d)) dx = max(dx, d);
+    if (__any(dw >= d)) dw = max(dw, d);
+  }
+  dx = __builtin_amdgcn_readfirstlane(dx);
+  dw = __builtin_amdgcn_readfirstlane(dw);
+
+  struct Chunk {
+    i32x4 a[2][2], b[2][2];  // [32-k step][32-row block]
+  };
+  for (int s = min(dx + dw - 2, kI8Digits - 1); s >= 0; --s) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) total[i][j][r] = (int32_t)((uint32_t)total[i][j][r] << 8);
+    for (int di = max(0, s - dw + 1); di <= min(s, dx - 1); ++di) {
+      const int dj = s - di;
+      const i32x4 rsrc_a = buffer_rsrc(
+          a.A8p + (int64_t)di * a.plane_x + (int64_t)(m0 >> 5) * block_bytes, 2 * (int64_t)block_bytes);
+      const i32x4 rsrc_b = buffer_rsrc(
+          a.B8p + (int64_t)dj * a.plane_w + (int64_t)(n0 >> 5) * block_bytes, 2 * (int64_t)block_bytes);
+      int cx = 0, cw = 0;
+      auto load = [&](Chunk& f, int t) __attribute__((always_inline)) {
+        if ((t & 63) == 0) {  // uniform: the counts of the next 64 chunks
+          const int u = min(t + lane, n - 1);
+          cx = fx[(int64_t)u * stride];
+          cw = fw[(int64_t)u * stride];
+        }
+        const bool in = t < n;
+        const int at = (first + t * stride) * 2048;  // the chunk's two fragments of a block
+        const int oa = in && __builtin_amdgcn_readlane(cx, t & 63) > di ? lane * 16 : kOutOfRange;
+        const int ob = in && __builtin_amdgcn_readlane(cw, t & 63) > dj ? lane * 16 : kOutOfRange;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            f.a[k][i] = raw_buffer_load_i32x4(rsrc_a, oa, in ? at + k * 1024 + i * block_bytes : 0, 0);
+            f.b[k][i] = raw_buffer_load_i32x4(rsrc_b, ob, in ? at + k * 1024 + i * block_bytes : 0, 0);
+          }
+      };
+      i32x16 acc[2][2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+      Chunk f[D];
+#pragma unroll
+      for (int d = 0; d < D; ++d) load(f[d], d);
+#pragma unroll 1
+      for (int t = 0; t < n; t += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+#pragma unroll
+          for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+              for (int j = 0; j < 2; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f[d].a[k][i], f[d].b[k][j], acc[i][j], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          load(f[d], t + d + D);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) total[i][j][r] = (int32_t)((uint32_t)total[i][j][r] + (uint32_t)acc[i][j][r]);
+    }
+  }
+}
+
+// Rows and columns of a 32x32 block's accumulator: lane holds rows 8*(r/4) +
+// 4*(lane/32) + r%4 and column lane%32, so each store writes two 128-byte row
+// segments. Elements past M or N are not stored.
+template <int EPI>
+__device__ __forceinline__ void store_block_checked(const GemmI32Args& a, const i32x16& v, int m0, int n0) {
+  const int lane = threadIdx.x & 63;
+  const int n = n0 + (lane & 31);
+  if (n >= a.N) return;
+  const int32_t b = epi_has_bias(EPI) ? a.bias[n] : 0;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int m = m0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+    if (m < a.M) __builtin_nontemporal_store(apply_epilogue_i32<EPI>(v[r], b), a.C + (int64_t)m * a.ldc + n);
+  }
+}
+
+// A 128x128 tile of a workgroup of four waves whose operands need more than
+// one digit: each wave a 64x64 quadrant over all of K.
+template <int EPI>
+__device__ __forceinline__ void digits_tile128(const GemmI32Args& a, int m0, int n0) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m = m0 + 64 * (wave & 1), n = n0 + 64 * (wave >> 1);
+  i32x16 total[2][2];
+  digits_wave<2>(a, m, n, 0, 1, total);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) store_block_checked<EPI>(a, total[i][j], m + 32 * i, n + 32 * j);
+}
+
+// 64x64 output tile per workgroup of four waves, each wave the whole tile over
+// every fourth 64-k chunk, the four totals summed through LDS (integer sums:
+// any order). For layers whose 128x128 tiles leave most CUs idle.
+template <int EPI>
+__global__ void __launch_bounds__(256, 2) gemm_i8_tile64_kernel(GemmI32Args a) {
+  __shared__ i32x4 red[4 * 16 * 64];  // [wave][block * 4 + q][lane]
+  int tm, tn;
+  tile_coords(blockIdx.x, a.tiles_m, a.tiles_n, tm, tn);
+  const int m0 = __builtin_amdgcn_readfirstlane(tm * 64), n0 = __builtin_amdgcn_readfirstlane(tn * 64);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  i32x16 total[2][2];
+  digits_wave<2>(a, m0, n0, wave, 4, total);
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const i32x16& v = total[b >> 1][b & 1];
+      red[(wave * 16 + b * 4 + q) * 64 + lane] = i32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+    }
+  __syncthreads();
+  // Wave w finishes block (w / 2, w % 2).
+  i32x16 sum;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    i32x4 v = red[(wave * 4 + q) * 64 + lane];
+#pragma unroll
+    for (int p = 1; p < 4; ++p) v += red[(p * 16 + wave * 4 + q) * 64 + lane];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sum[4 * q + e] = v[e];
+  }
+  store_block_checked<EPI>(a, sum, m0 + 32 * (wave >> 1), n0 + 32 * (wave & 1));
 }
 
 // ------------------------------------------------- exact i32 vector-ALU tile
@@ -163,12 +374,10 @@ struct ValuSmem {
   uint32_t w[kValuK][kValuTile + 1];
 };
 
-// NT threads stage the operands; the first 256 compute (8x8 outputs each).
-template <int EPI, int NT>
+template <int EPI>
 __device__ void valu_tile_i32(const GemmI32Args& a, int m0, int n0, ValuSmem& sm) {
   const int tid = threadIdx.x;
-  const bool computes = tid < 256;
-  const int ty = (tid & 255) / 16, tx = tid % 16;
+  const int ty = tid / 16, tx = tid % 16;
   uint32_t acc[8][8];
 #pragma unroll
   for (int i = 0; i < 8; ++i)
@@ -176,19 +385,19 @@ __device__ void valu_tile_i32(const GemmI32Args& a, int m0, int n0, ValuSmem& sm
     for (int j = 0; j < 8; ++j) acc[i][j] = 0u;
 
   for (int k0 = 0; k0 < a.K; k0 += kValuK) {
-    for (int idx = tid; idx < kValuTile * kValuK; idx += NT) {
+    for (int idx = tid; idx < kValuTile * kValuK; idx += 256) {
       const int r = idx / kValuK, c = idx % kValuK;
       const int m = m0 + r, k = k0 + c;
       sm.x[r][c] = (m < a.M && k < a.K) ? (uint32_t)a.X[(int64_t)m * a.ldx + k] : 0u;
     }
-    for (int idx = tid; idx < kValuK * kValuTile; idx += NT) {
+    for (int idx = tid; idx < kValuK * kValuTile; idx += 256) {
       const int r = idx / kValuTile, c = idx % kValuTile;
       const int k = k0 + r, n = n0 + c;
       sm.w[r][c] = (k < a.K && n < a.N) ? (uint32_t)a.W[(int64_t)k * a.ldw + n] : 0u;
     }
     __syncthreads();
 #pragma unroll 4
-    for (int kk = 0; kk < (computes ? kValuK : 0); ++kk) {
+    for (int kk = 0; kk < kValuK; ++kk) {
       uint32_t xv[8], wv[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) xv[i] = sm.x[ty + 16 * i][kk];
@@ -201,7 +410,6 @@ __device__ void valu_tile_i32(const GemmI32Args& a, int m0, int n0, ValuSmem& sm
     }
     __syncthreads();
   }
-  if (!computes) return;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int m = m0 + ty + 16 * i;
@@ -220,7 +428,7 @@ template <int EPI>
 __global__ void __launch_bounds__(256) gemm_i32_valu_kernel(GemmI32Args a) {
   __shared__ ValuSmem sm;
   const int tm = blockIdx.x / a.tiles_n, tn = blockIdx.x % a.tiles_n;
-  valu_tile_i32<EPI, 256>(a, tm * kValuTile, tn * kValuTile, sm);
+  valu_tile_i32<EPI>(a, tm * kValuTile, tn * kValuTile, sm);
 }
 
 // -------------------------------------------------------- int8 MFMA kernel
@@ -236,13 +444,12 @@ __global__ void __launch_bounds__(256) gemm_i32_valu_kernel(GemmI32Args a) {
 // pair the same k.
 template <int EPI, int D>
 __global__ void __launch_bounds__(256) gemm_i8_kernel(GemmI32Args a) {
-  __shared__ ValuSmem valu;
   int tm, tn;
   tile_coords(blockIdx.x, a.tiles_m, a.tiles_n, tm, tn);
   const int m0 = tm * kI8Tile, n0 = tn * kI8Tile;
 
-  if (tile_out_of_range<256>(a, m0, n0)) {  // some value outside int8: exact i32 path
-    valu_tile_i32<EPI, 256>(a, m0, n0, valu);
+  if (tile_is_wide<256>(a, m0, n0)) {  // some value outside int8
+    digits_tile128<EPI>(a, m0, n0);
     return;
   }
 
@@ -344,13 +551,12 @@ template <int EPI, int D>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 gemm_i8_ksplit_kernel(GemmI32Args a) {
   __shared__ i32x4 red[kI8KsRedBytes / 16];
-  static_assert(sizeof(ValuSmem) <= sizeof(red), "exact-path staging must fit the reduce buffer");
   int tm, tn;
   tile_coords(blockIdx.x, a.tiles_m, a.tiles_n, tm, tn);
   const int m0 = tm * kI8Tile, n0 = tn * kI8Tile;
 
-  if (tile_out_of_range<256>(a, m0, n0)) {  // some value outside int8: exact i32 path
-    valu_tile_i32<EPI, 256>(a, m0, n0, *reinterpret_cast<ValuSmem*>(red));
+  if (tile_is_wide<256>(a, m0, n0)) {  // some value outside int8
+    digits_tile128<EPI>(a, m0, n0);
     return;
   }
 
@@ -556,6 +762,15 @@ hipError_t launch_gemm_i8(int epi, GemmI32Args a, hipStream_t stream, int varian
     case 8: return launch_i8_depth<false, 8>(epi, a, stream);
     default: return hipErrorInvalidValue;
   }
+}
+
+hipError_t launch_gemm_i8_tile64(int epi, GemmI32Args a, hipStream_t stream) {
+  if (a.M <= 0 || a.N <= 0 || a.K <= 0 || a.Kp % kI8Tile || a.Kp < a.K) return hipErrorInvalidValue;
+  a.tiles_m = (a.M + 63) / 64;
+  a.tiles_n = (a.N + 63) / 64;
+  const dim3 grid(a.tiles_m * a.tiles_n);
+  EDSL_I32_EPI_SWITCH(gemm_i8_tile64_kernel, grid, a)
+  return hipGetLastError();
 }
 
 hipError_t launch_gemm_i32_valu(int epi, GemmI32Args a, hipStream_t stream) {

@@ -103,38 +103,44 @@ constexpr int kGemvMaxM = 64;
 // v_mfma_i32_32x32x32_i8 operand of that block, one 16-byte load per lane.
 // The packed copies cover M, N, K rounded up to multiples of kI8Tile (Mp, Np,
 // Kp); elements past the real M, N or K are zero, so they add nothing.
+// Values outside int8 take more than one copy: plane d holds digit d of the
+// signed base-256 digits (v = sum_d 256^d digit_d modulo 2^32), planes Mp*Kp
+// (X) or Np*Kp (W) bytes apart.
 struct NarrowI8Args {
   const int32_t* X;   // [M][K], ldx
   const int32_t* W;   // [K][N], ldw
-  int8_t* X8p;        // X narrowed, fragment-packed over (Mp, Kp)
-  int8_t* W8p;        // W narrowed, fragment-packed over (Np, Kp) (W transposed)
+  int8_t* X8p;        // X narrowed, fragment-packed over (Mp, Kp), kI8Digits planes
+  int8_t* W8p;        // W narrowed, fragment-packed over (Np, Kp) (W transposed), kI8Digits planes
   int64_t ldx, ldw;
   int M, N, K;        // real sizes
   int Mp, Np, Kp;     // padded sizes (multiples of kI8Tile)
-  // Range flags, one byte per 64x64 tile, all written on every call: 1 when the
-  // tile holds a value outside [-128, 127], else 0. X: [Mp/64][Kp/64]; W:
+  // Digit counts, one byte per 64x64 tile, all written on every call: 1 when
+  // every value of the tile lies in [-128, 127], up to kI8Digits; a tile's
+  // planes past its count are not written. X: [Mp/64][Kp/64]; W:
   // [Np/64][Kp/64] (indexed by W's column tile, then its k tile).
   uint8_t* flags_x;
   uint8_t* flags_w;
 };
 
 struct GemmI32Args {
-  const int8_t* A8p;  // fragment-packed X (int8 fast path)
-  const int8_t* B8p;  // fragment-packed W^T (int8 fast path)
-  const int32_t* X;   // [M][K], ldx   (exact i32 fallback)
-  const int32_t* W;   // [K][N], ldw   (exact i32 fallback)
+  const int8_t* A8p;  // fragment-packed X (int8 path), plane 0
+  const int8_t* B8p;  // fragment-packed W^T (int8 path), plane 0
+  int64_t plane_x, plane_w;  // bytes from one digit plane to the next
+  const int32_t* X;   // [M][K], ldx   (vector-ALU path)
+  const int32_t* W;   // [K][N], ldw   (vector-ALU path)
   const int32_t* bias;
   int32_t* C;         // [M][N], ldc
   int64_t ldx, ldw, ldc;
   int M, N, K;
   int Kp;             // K of the packed copies (int8 path; a multiple of kI8Tile)
   int tiles_m, tiles_n;
-  // Range flags of the narrowing pass (int8 path): a tile takes the exact i32
-  // path when a flag of its X row panels or W column panels is set.
+  // Digit counts of the narrowing pass (int8 path): a tile runs the products
+  // of as many planes as its X row panels and W column panels need.
   const uint8_t* flags_x;
   const uint8_t* flags_w;
 };
 
+constexpr int kI8Digits = 4;   // signed base-256 digits of an i32, modulo 2^32
 constexpr int kI8Tile = 128;   // tile of the int8 MFMA path; packed copies are padded to it
 hipError_t launch_narrow_i8(NarrowI8Args args, hipStream_t stream);
 // variant = wave layout + fragment prefetch depth in 32-k steps:
@@ -148,6 +154,8 @@ constexpr int kI8DefaultVariant = 3;
 int gemm_i8_depth(int variant, int K);
 const char* gemm_i8_layout(int variant);
 hipError_t launch_gemm_i8(int epi, GemmI32Args args, hipStream_t stream, int variant = -1);
+// 64x64 tiles, K split over the four waves of a workgroup.
+hipError_t launch_gemm_i8_tile64(int epi, GemmI32Args args, hipStream_t stream);
 // Exact wrapping i32 GEMM on the vector ALUs: any shape, any alignment.
 hipError_t launch_gemm_i32_valu(int epi, GemmI32Args args, hipStream_t stream);
 

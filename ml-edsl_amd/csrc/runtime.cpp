@@ -508,8 +508,9 @@ void launch_i32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream) {
   a.M = (int)L.M;
   a.N = (int)L.N;
   a.K = (int)L.K;
-  // The int8 path is exact for K < 2^17 (each product of int8 values has
-  // magnitude <= 2^14, so no i32 partial sum can overflow). Its packed copies
+  // The int8 path is exact for K < 2^17 (each product of two signed base-256
+  // digits has magnitude <= 2^14, so no i32 sum over K can overflow; values
+  // outside int8 take several digits). Its packed copies
   // are padded with zeros to multiples of the 128-wide tile, so any M, N and
   // K run on it; only the stores are limited to the real M x N.
   const bool tiled = a.M > 0 && a.N > 0 && a.K > 0 && a.K < (1 << 17);
@@ -518,9 +519,9 @@ void launch_i32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream) {
     const int Mp = pad(a.M), Np = pad(a.N), Kp = pad(a.K);
     a.Kp = Kp;
     const size_t xs = (size_t)Mp * Kp, ws = (size_t)Np * Kp;
-    int8_t* x8 = static_cast<int8_t*>(ds.i8_x.ensure(xs, false));
-    int8_t* w8 = static_cast<int8_t*>(ds.i8_w.ensure(ws, false));
-    // One range flag per 64x64 tile of the padded X and W (rewritten by every call).
+    int8_t* x8 = static_cast<int8_t*>(ds.i8_x.ensure(kI8Digits * xs, false));
+    int8_t* w8 = static_cast<int8_t*>(ds.i8_w.ensure(kI8Digits * ws, false));
+    // One digit count per 64x64 tile of the padded X and W (rewritten by every call).
     const size_t fx = (size_t)(Mp / 64) * (Kp / 64), fw = (size_t)(Np / 64) * (Kp / 64);
     uint8_t* flags = static_cast<uint8_t*>(ds.i8_flags.ensure(fx + fw, false));
     NarrowI8Args n{};
@@ -542,14 +543,27 @@ void launch_i32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream) {
     check_hip(launch_narrow_i8(n, stream), "narrow_i8 launch");
     a.A8p = x8;
     a.B8p = w8;
+    a.plane_x = (int64_t)xs;
+    a.plane_w = (int64_t)ws;
     a.flags_x = flags;
     a.flags_w = flags + fx;
+    const int tiles = (Mp / kI8Tile) * (Np / kI8Tile);
+    // 64x64 tiles where 128x128 ones give at most half of the CUs a workgroup
+    // (int8 values, then X values of up to 1000, us on 64x64 against 128x128:
+    // 512x1024x512 9.8 against 12.0 and 12.9 against 25.2, 1024^3 11.3 / 13.6
+    // and 14.3 / 27.7, 2048x1024x1024, exactly half, 13.8 / 14.5 and 18.6 /
+    // 28.3; above it they lose on int8 values: 1536x1024x1536 18.5 / 15.6).
+    if (g_force_i8 < 0 && 2 * tiles <= ds.cus) {
+      check_hip(launch_gemm_i8_tile64(epi, a, stream), "gemm_i8 launch");
+      scratch_end(ds, stream);
+      set_plan("narrow_i8+gemm_i8 tile=64x64 waves=ksplit grid=%d", ((a.M + 63) / 64) * ((a.N + 63) / 64));
+      return;
+    }
     const int variant = (g_force_i8 >= 0 && g_force_i8 < kI8Variants) ? g_force_i8 : kI8DefaultVariant;
     check_hip(launch_gemm_i8(epi, a, stream, variant), "gemm_i8 launch");
     scratch_end(ds, stream);
     set_plan("narrow_i8+gemm_i8 variant=%d waves=%s depth=%d grid=%d", variant, gemm_i8_layout(variant),
-             gemm_i8_depth(variant, Kp),
-             (Mp / kI8Tile) * (Np / kI8Tile));
+             gemm_i8_depth(variant, Kp), tiles);
   } else {
     check_hip(launch_gemm_i32_valu(epi, a, stream), "gemm_i32_valu launch");
     set_plan("gemm_i32_valu grid=%d", ((a.M + 127) / 128) * ((a.N + 127) / 128));
