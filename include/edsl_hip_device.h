@@ -92,8 +92,8 @@ int edsl_hip_dense_i32_launch(const int32_t *X, int64_t ldx, const int32_t *W, i
 /* Description of the kernels the calling thread's last call launched, e.g.
  * "gemm_f32 cfg=f32_256x256x16_w4x4 grid=256" (a "_edge" suffix: partial
  * edge tiles), "gemv_f32 mb=1 ksplit=4 cols=128 grid=256 +reduce" (with
- * "+xunaligned": X rows read with 4-byte loads; "+ktail": the reduce kernel adds
- * the last K % 16 rows) or "narrow_i8+gemm_i8 variant=3 waves=ksplit depth=2
+ * "+xunaligned", "+wrealigned", "+wunaligned": rows of X or W that are not
+ * 16-byte aligned; "+ktail": the reduce kernel adds the last K % 16 rows) or "narrow_i8+gemm_i8 variant=3 waves=ksplit depth=2
  * grid=256"; returns its length. */
 int edsl_hip_last_plan(char *buf, size_t len);
 

@@ -45,7 +45,10 @@
 namespace edsl {
 namespace {
 
-typedef float f32x3 __attribute__((ext_vector_type(3)));
+// Vectors of floats at any 4-byte aligned address (the vector loads and stores
+// of gfx950 need no more than that).
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 
 // Waves per workgroup for MB row blocks of 16 and WN waves side by side.
 constexpr int waves_per_wg(int mb, int wn) { return (mb == 1 ? 4 : 8) > wn ? (mb == 1 ? 4 : 8) : wn; }
@@ -65,22 +68,22 @@ __device__ __forceinline__ float epilogue_rt(float acc, float b, float alpha, in
   }
 }
 
-// XV: X rows are 16-byte aligned (row stride % 4 == 0) and are read with one
-// 16-byte load per row block and step; otherwise with four 4-byte loads
-// (X is small and read from the caches, so this costs little against W).
-// WM (GemvF32Args::w_mode): kWVector -- W, Y and the bias are 16-byte
-// aligned, their row strides and N multiples of 4: a lane's CPL columns are
-// one vector load or store, all in or all out of range. Otherwise Y and the
-// bias are 4-byte accesses and columns past N are not stored; W is read
-// either with a 4-byte load per column (kWScalar; columns past N read column
-// N - 1) or, for CPL = 4, realigned (kWRealign): the lane's 4 columns lie in
-// two neighbouring 16-byte chunks of the row, loaded whole (the second mostly
-// by the neighbouring lane), and a select by the row's offset within its
-// chunk picks them; the caller leaves the last row of W to the K tail.
-template <int MB, int CPL, int WN, bool XV, int WM>
+// WM (GemvF32Args::w_mode): kWVector and kWShared (N >= 4) -- a lane's CPL
+// columns are one vector load per row, whatever the alignment of W and its row
+// stride; a lane whose columns reach past N loads the last CPL columns instead
+// and stores only its own of them. kWScalar (N < 4): a 4-byte load per column,
+// columns past N reading column N - 1. X rows are read with one 16-byte load
+// per row block and step, at any alignment too.
+// kWVector is for W rows that start on 128-byte lines: every line belongs to
+// one workgroup and is streamed past the caches (16x8192x8192 44.5 us against
+// 50.6 us with plain loads). Otherwise a row's line at a block edge is also
+// read by the neighbouring block: plain loads, and neighbours on one XCD and
+// its L2 (16x4096x4097 21.4 us against 25.2 us streamed in launch order, and
+// 30.2 us for the aligned chunks realigned in registers that this replaced).
+template <int MB, int CPL, int WN, int WM>
 __global__ void __launch_bounds__(waves_per_wg(MB, WN) * 64)
 gemv_f32_kernel(GemvF32Args a, int epi) {
-  using vec = typename std::conditional<CPL == 4, f32x4, f32x2>::type;
+  using vec = typename std::conditional<CPL == 4, f32x4u, f32x2u>::type;
   constexpr int NW = waves_per_wg(MB, WN);
   static_assert(NW % WN == 0, "waves side by side must divide the workgroup");
   constexpr int WK = NW / WN;
@@ -98,8 +101,15 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
   const int wn = wave % WN;
   const int wk = wave / WN;
   const int groups = (a.N + kGroupCols - 1) / kGroupCols;  // the last may be partial
-  const int g = blockIdx.x % groups;
-  const int split = blockIdx.x / groups;
+  int wg = blockIdx.x;
+  if constexpr (WM == kWShared) {
+    // Workgroup w runs on XCD w % 8: give each XCD a run of neighbouring
+    // column blocks (the first total % 8 XCDs have one more).
+    const int total = groups * a.ksplit, x = wg % 8;
+    wg = x * (total / 8) + min(x, total % 8) + wg / 8;
+  }
+  const int g = wg % groups;
+  const int split = wg / groups;
   const int n0 = g * kGroupCols + kWaveCols * wn;
   // K, in 16-row chunks, is spread as evenly as possible over the ksplit x WK
   // slices: slice i = split * WK + wk takes chunks [i*C/S, (i+1)*C/S). When S
@@ -119,69 +129,17 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
     for (int c = 0; c < CPL; ++c) acc[mb][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   const int64_t ldw = a.ldw;
-  // kWVector: lanes whose columns lie past N (a partial last column block)
-  // read the last CPL columns instead; their results are never stored. N % 4
-  // == 0, so a lane's CPL columns are all in or all out. kWScalar: wbase is
-  // the row start and cofs the lane's columns, each clamped to N - 1.
-  static_assert(WM != kWRealign || CPL == 4, "realigned W rows need 4 columns per lane");
-  // Realigned rows: every lane's column offset and every step's row offset
-  // within the wave's slice are multiples of 4, so the offset of a row within
-  // its 16-byte chunk depends only on the row's slot s = q % 4 in the step:
-  // dsh[s], the same for every lane and step.
-  //
-  // A lane loads one chunk per row, the one holding its first column. The next chunk, which holds the rest, is
-  // its right neighbour's, taken with a row shift (lanes 16g .. 16g+15 share
-  // a row); only lane 16g+15 has no neighbour and loads it as well (the other
-  // lanes masked off; 12 bytes, the most it needs). Both are kept until just
-  // before the MFMAs that read them, so a wave's loads stay in flight. Lanes
-  // wholly past N read the chunk at r4 = N rounded up to 4, the one after the
-  // last lane that holds a column below N, so that its neighbour finds the
-  // right chunk there. Every chunk loaded holds a column below N of its row or
-  // one of the next row's first elements (the caller leaves the last row of W
-  // to the K tail), so no load leaves the matrix's pages.
-  constexpr bool kDefer = WM == kWRealign;
   const int col_lane = n0 + CPL * li;
-  const int r4 = (a.N + 3) & ~3;
-  const int col_w = WM == kWVector ? min(col_lane, a.N - CPL) : kDefer ? min(col_lane, r4) : 0;
+  const int col_w = WM != kWScalar ? min(col_lane, a.N - CPL) : 0;
   const float* wbase = a.W + (int64_t)(kbeg + 4 * lg) * ldw + col_w;
   int cofs[CPL];
 #pragma unroll
   for (int c = 0; c < CPL; ++c) cofs[c] = min(col_lane + c, a.N - 1);
-  int dsh[4];
-#pragma unroll
-  for (int s = 0; s < 4; ++s)
-    dsh[s] = (int)(((reinterpret_cast<uintptr_t>(a.W) >> 2) + (uint64_t)s * (uint64_t)ldw) & 3);
-  // Lane 16g+15 loads its second chunk when it holds a column below N.
-  const bool own_next = li == 15 && col_lane < a.N;
-  // Elements d .. d+3 (d = dsh[s]) of the lane's chunk c0 and the next one.
-  // The row shift runs on every lane (a lane masked off would read as
-  // invalid to its neighbour); the selects follow.
-  auto realign = [&](const f32x4& c0, const f32x3& own, int s) {
-    auto shl1 = [](float v) {  // lane i <- lane i + 1 of its row of 16
-      return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x101, 0xf, 0xf, false));
-    };
-    const f32x3 next{shl1(c0[0]), shl1(c0[1]), shl1(c0[2])};
-    const f32x3 c1 = li == 15 ? own : next;
-    const bool b0 = dsh[s] & 1, b1 = dsh[s] & 2;
-    const float t0 = b0 ? c0[1] : c0[0], t1 = b0 ? c0[2] : c0[1], t2 = b0 ? c0[3] : c0[2];
-    const float t3 = b0 ? c1[0] : c0[3], t4 = b0 ? c1[1] : c1[0], t5 = b0 ? c1[2] : c1[1];
-    return f32x4{b1 ? t2 : t0, b1 ? t3 : t1, b1 ? t4 : t2, b1 ? t5 : t3};
-  };
-  // The second chunk is loaded as 12 bytes, so no register of an outstanding
-  // load is dead (a dead one is reused as a temporary, and the wave then
-  // waits for the load before the temporary is written).
-  struct Chunks { f32x4 c0; f32x3 c1; };
-  using wreg = typename std::conditional<kDefer, Chunks, vec>::type;
-  auto load_row = [&](const float* row, int s) {
+  auto load_row = [&](const float* row) {
     if constexpr (WM == kWVector) {
       return __builtin_nontemporal_load(reinterpret_cast<const vec*>(row));
-    } else if constexpr (kDefer) {
-      const f32x4* p0 = reinterpret_cast<const f32x4*>(row - dsh[s]);
-      Chunks r;
-      r.c0 = __builtin_nontemporal_load(p0);
-      r.c1 = f32x3{0.0f, 0.0f, 0.0f};
-      if (own_next && dsh[s] != 0) r.c1 = __builtin_nontemporal_load(reinterpret_cast<const f32x3*>(p0 + 1));
-      return r;
+    } else if constexpr (WM == kWShared) {
+      return *reinterpret_cast<const vec*>(row);
     } else {
       vec v;
 #pragma unroll
@@ -205,7 +163,7 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
     constexpr int U = sizeof(w) / sizeof(w[0]) / 4;
     const float* wp = wbase + (int64_t)k * ldw;
 #pragma unroll
-    for (int q = 0; q < 4 * U; ++q) w[q] = load_row(wp + (int64_t)(16 * (q / 4) + q % 4) * ldw, q % 4);
+    for (int q = 0; q < 4 * U; ++q) w[q] = load_row(wp + (int64_t)(16 * (q / 4) + q % 4) * ldw);
   };
   auto load_x = [&](auto& x, int k) {
     constexpr int U = sizeof(x) / sizeof(x[0]);
@@ -213,19 +171,11 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
-        const float* p = xp[mb] + k + 16 * u;
-        if constexpr (XV)
-          x[u][mb] = *reinterpret_cast<const f32x4*>(p);
-        else
-          x[u][mb] = f32x4{p[0], p[1], p[2], p[3]};
+        const f32x4u v = *reinterpret_cast<const f32x4u*>(xp[mb] + k + 16 * u);
+        x[u][mb] = f32x4{v[0], v[1], v[2], v[3]};
       }
   };
-  auto mfma_q = [&](const f32x4 (&xu)[MB], int s, const wreg& wr) {
-    vec wq;
-    if constexpr (kDefer)
-      wq = realign(wr.c0, wr.c1, s);
-    else
-      wq = wr;
+  auto mfma_q = [&](const f32x4 (&xu)[MB], int s, const vec& wq) {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -246,7 +196,7 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
   const int nit = kwave / (16 * kU);
   const int r0 = nit > 0 ? (int)(((unsigned)blockIdx.x * 2654435761u >> 8) + (unsigned)wk * 977u) % nit : 0;
   if (nit > 0) {
-    wreg w[4 * kU];
+    vec w[4 * kU];
     f32x4 x[kU][MB], xn[kU][MB];
     int it = r0;
     load_x(x, it * 16 * kU);
@@ -260,7 +210,7 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
 #pragma unroll
       for (int q = 0; q < 4 * kU; ++q) {
         mfma_q(x[q / 4], q % 4, w[q]);
-        w[q] = load_row(wp + (int64_t)(16 * (q / 4) + q % 4) * ldw, q % 4);
+        w[q] = load_row(wp + (int64_t)(16 * (q / 4) + q % 4) * ldw);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
@@ -274,7 +224,7 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
   }
   // Remaining single steps (kwave not a multiple of 16*kU).
   for (int k = nit * 16 * kU; k < kwave; k += 16) {
-    wreg w[4];
+    vec w[4];
     f32x4 x[1][MB];
     load_x(x, k);
     load_w(w, k);
@@ -304,19 +254,32 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
     if (wk != 0) return;
   }
 
-  // Lane holds rows 16*mb + 4*lg + r and columns n0 + CPL*li + c.
-  const int col = n0 + CPL * li;
-  if (col >= a.N) return;
+  // Lane holds rows 16*mb + 4*lg + r; register c is column col_lane + c, or
+  // col_w + c on a lane whose columns reach past N: such a lane stores its
+  // own columns only, one by one (a neighbour's workgroup walks K in another
+  // order, so the others could differ in their last bits).
+  if (col_lane >= a.N) return;
+  const bool full = col_lane + CPL <= a.N;
+  const int own = WM != kWScalar ? col_lane - col_w : 0;  // first register of an own column
+  auto store = [&](float* row, const vec& v) {
+    if (full) {
+      *reinterpret_cast<vec*>(row + col_lane) = v;
+    } else {
+#pragma unroll
+      for (int c = 0; c < CPL; ++c)
+        if (c >= own && col_lane + c - own < a.N) row[col_lane + c - own] = v[c];
+    }
+  };
   if (a.ksplit == 1) {
     vec bv;
 #pragma unroll
     for (int c = 0; c < CPL; ++c) bv[c] = 0.0f;
     if (epi_has_bias(epi)) {
-      if constexpr (WM == kWVector) {
-        bv = *reinterpret_cast<const vec*>(a.bias + col);
+      if constexpr (WM != kWScalar) {
+        bv = *reinterpret_cast<const vec*>(a.bias + col_w);
       } else {
 #pragma unroll
-        for (int c = 0; c < CPL; ++c) bv[c] = col + c < a.N ? a.bias[col + c] : 0.0f;
+        for (int c = 0; c < CPL; ++c) bv[c] = a.bias[cofs[c]];
       }
     }
 #pragma unroll
@@ -328,14 +291,7 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
           vec y;
 #pragma unroll
           for (int c = 0; c < CPL; ++c) y[c] = epilogue_rt(acc[mb][c][r], bv[c], a.alpha, epi);
-          float* dst = a.Y + (int64_t)row * a.ldy + col;
-          if constexpr (WM == kWVector) {
-            *reinterpret_cast<vec*>(dst) = y;
-          } else {
-#pragma unroll
-            for (int c = 0; c < CPL; ++c)
-              if (col + c < a.N) dst[c] = y[c];
-          }
+          store(a.Y + (int64_t)row * a.ldy, y);
         }
       }
     return;
@@ -350,7 +306,7 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
         vec p;
 #pragma unroll
         for (int c = 0; c < CPL; ++c) p[c] = acc[mb][c][r];
-        *reinterpret_cast<vec*>(a.partials + ((int64_t)split * prow + row) * a.ldp + col) = p;
+        store(a.partials + ((int64_t)split * prow + row) * a.ldp, p);
       }
     }
 }
@@ -358,19 +314,19 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
 // Y[m, 4j..4j+3] = epilogue(sum over splits s = 0..ksplit-1, in order, plus
 // the K tail rows).
 // All split loads are issued before the first add so their latencies overlap.
-// WV as for gemv_f32_kernel: otherwise the bias, the tail rows of W and Y
-// are 4-byte accesses, columns past N neither read nor written. The partials
-// always have an aligned row pitch (ldp, a multiple of 4).
+// W, the bias and Y may have any alignment; the last four columns of a row
+// that N cuts short are read and written one by one. The partials always have
+// an aligned row pitch (ldp, a multiple of 4).
 // One wave per workgroup spreads the reduction over more CUs than 256-thread
 // workgroups (the c4 column shard: 16 workgroups of 256 threads); measured
 // 0.2 us faster per layer at c4 and at its column shard.
-template <bool WV>
 __global__ void __launch_bounds__(64) gemv_reduce_kernel(GemvF32Args a, int epi, int prow) {
   const int64_t idx = (int64_t)blockIdx.x * 64 + threadIdx.x;  // over M * ceil(N/4)
   const int n4 = (a.N + 3) / 4;
   if (idx >= (int64_t)a.M * n4) return;
   const int row = (int)(idx / n4);
   const int col = 4 * (int)(idx % n4);
+  const bool full = col + 4 <= a.N;
   f32x4 v[kMaxSplit];
 #pragma unroll
   for (int sp = 0; sp < kMaxSplit; ++sp)
@@ -379,8 +335,9 @@ __global__ void __launch_bounds__(64) gemv_reduce_kernel(GemvF32Args a, int epi,
           reinterpret_cast<const f32x4*>(a.partials + ((int64_t)sp * prow + row) * a.ldp + col));
   f32x4 bv = {0.0f, 0.0f, 0.0f, 0.0f};
   if (epi_has_bias(epi)) {
-    if constexpr (WV) {
-      bv = *reinterpret_cast<const f32x4*>(a.bias + col);
+    if (full) {
+      const f32x4u v4 = *reinterpret_cast<const f32x4u*>(a.bias + col);
+      bv = f32x4{v4[0], v4[1], v4[2], v4[3]};
     } else {
 #pragma unroll
       for (int c = 0; c < 4; ++c) bv[c] = col + c < a.N ? a.bias[col + c] : 0.0f;
@@ -401,8 +358,9 @@ __global__ void __launch_bounds__(64) gemv_reduce_kernel(GemvF32Args a, int epi,
       const int k = min(a.K + t, a.k_end - 1);
       xt[t] = a.x_tail[(int64_t)row * a.ldx_tail + k];
       const float* wr = a.W + (int64_t)k * a.ldw + col;
-      if constexpr (WV) {
-        wt[t] = *reinterpret_cast<const f32x4*>(wr);
+      if (full) {
+        const f32x4u v4 = *reinterpret_cast<const f32x4u*>(wr);
+        wt[t] = f32x4{v4[0], v4[1], v4[2], v4[3]};
       } else {
 #pragma unroll
         for (int c = 0; c < 4; ++c) wt[t][c] = col + c < a.N ? wr[c] : 0.0f;
@@ -416,8 +374,8 @@ __global__ void __launch_bounds__(64) gemv_reduce_kernel(GemvF32Args a, int epi,
 #pragma unroll
   for (int c = 0; c < 4; ++c) y[c] = epilogue_rt(s[c], bv[c], a.alpha, epi);
   float* dst = a.Y + (int64_t)row * a.ldy + col;
-  if constexpr (WV) {
-    *reinterpret_cast<f32x4*>(dst) = y;
+  if (full) {
+    *reinterpret_cast<f32x4u*>(dst) = f32x4u{y[0], y[1], y[2], y[3]};
   } else {
 #pragma unroll
     for (int c = 0; c < 4; ++c)
@@ -425,35 +383,26 @@ __global__ void __launch_bounds__(64) gemv_reduce_kernel(GemvF32Args a, int epi,
   }
 }
 
-template <int MB, bool XV, int WM>
-hipError_t launch_mb_x(int cols, int epi, const GemvF32Args& a, hipStream_t stream) {
+template <int MB, int WM>
+hipError_t launch_mb_w(int cols, int epi, const GemvF32Args& a, hipStream_t stream) {
   const dim3 grid(((a.N + cols - 1) / cols) * a.ksplit);
   auto block = [](int wn) { return dim3(waves_per_wg(MB, wn) * 64); };
-  // Two columns per lane take 4-byte W loads where four would be realigned.
-  constexpr int WM2 = WM == kWRealign ? kWScalar : WM;
   switch (cols) {
-    case 32: hipLaunchKernelGGL((gemv_f32_kernel<MB, 2, 1, XV, WM2>), grid, block(1), 0, stream, a, epi); break;
-    case 64: hipLaunchKernelGGL((gemv_f32_kernel<MB, 4, 1, XV, WM>), grid, block(1), 0, stream, a, epi); break;
-    case 128: hipLaunchKernelGGL((gemv_f32_kernel<MB, 4, 2, XV, WM>), grid, block(2), 0, stream, a, epi); break;
-    case 256: hipLaunchKernelGGL((gemv_f32_kernel<MB, 4, 4, XV, WM>), grid, block(4), 0, stream, a, epi); break;
+    case 32: hipLaunchKernelGGL((gemv_f32_kernel<MB, 2, 1, WM>), grid, block(1), 0, stream, a, epi); break;
+    case 64: hipLaunchKernelGGL((gemv_f32_kernel<MB, 4, 1, WM>), grid, block(1), 0, stream, a, epi); break;
+    case 128: hipLaunchKernelGGL((gemv_f32_kernel<MB, 4, 2, WM>), grid, block(2), 0, stream, a, epi); break;
+    case 256: hipLaunchKernelGGL((gemv_f32_kernel<MB, 4, 4, WM>), grid, block(4), 0, stream, a, epi); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
-}
-
-
-template <int MB, int WM>
-hipError_t launch_mb_w(int cols, int epi, const GemvF32Args& a, hipStream_t stream) {
-  const bool xv = reinterpret_cast<uintptr_t>(a.X) % 16 == 0 && a.ldx % 4 == 0;
-  return xv ? launch_mb_x<MB, true, WM>(cols, epi, a, stream) : launch_mb_x<MB, false, WM>(cols, epi, a, stream);
 }
 
 template <int MB>
 hipError_t launch_mb(int cols, int epi, const GemvF32Args& a, hipStream_t stream) {
   switch (a.w_mode) {
     case kWVector: return launch_mb_w<MB, kWVector>(cols, epi, a, stream);
+    case kWShared: return launch_mb_w<MB, kWShared>(cols, epi, a, stream);
     case kWScalar: return launch_mb_w<MB, kWScalar>(cols, epi, a, stream);
-    case kWRealign: return launch_mb_w<MB, kWRealign>(cols, epi, a, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -465,15 +414,9 @@ int gemv_f32_waves_k(int cols, int M) {
   return waves_per_wg((M + 15) / 16, wn) / wn;
 }
 
-int gemv_f32_w_mode(const GemvF32Args& a) {
-  if (gemv_f32_vector_rows(a)) return kWVector;
-  return a.N >= 4 ? kWRealign : kWScalar;
-}
-
-bool gemv_f32_vector_rows(const GemvF32Args& a) {
-  auto al16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  return al16(a.W) && al16(a.Y) && (a.bias == nullptr || al16(a.bias)) && a.ldw % 4 == 0 && a.ldy % 4 == 0 &&
-         a.N % 4 == 0;
+int gemv_f32_w_mode(const float* W, int64_t ldw, int N) {
+  if (N < 4) return kWScalar;
+  return reinterpret_cast<uintptr_t>(W) % 128 == 0 && ldw % 32 == 0 ? kWVector : kWShared;
 }
 int gemv_f32_max_ksplit() { return kMaxSplit; }
 
@@ -491,10 +434,7 @@ hipError_t launch_gemv_f32(int epi, int cols, GemvF32Args a, hipStream_t stream)
   if (e != hipSuccess || a.ksplit == 1) return e;
   const int64_t items = (int64_t)a.M * ((a.N + 3) / 4);
   const dim3 g((unsigned)((items + 63) / 64));
-  if (a.w_mode == kWVector)
-    hipLaunchKernelGGL(gemv_reduce_kernel<true>, g, dim3(64), 0, stream, a, epi, 16 * mb);
-  else
-    hipLaunchKernelGGL(gemv_reduce_kernel<false>, g, dim3(64), 0, stream, a, epi, 16 * mb);
+  hipLaunchKernelGGL(gemv_reduce_kernel, g, dim3(64), 0, stream, a, epi, 16 * mb);
   return hipGetLastError();
 }
 

@@ -299,25 +299,27 @@ void check_dims(int64_t M, int64_t N, int64_t K) {
 }
 
 // Small-M plan. Widths are tried in the order 128, 256, 64, 32 columns per
-// workgroup; for each, the K split is the smallest power of two that gives at
-// least one workgroup per CU (every wave keeping >= 2 steps of 16 rows). The
-// first width that fills the chip is taken; when none does, the plan with the
-// most workgroups. The order is measured (M=16, K=N=8192 on MI355X): 128
-// columns x 4 splits beat 256 x 8 (more partial traffic), 64 x 2 (256-byte row
-// runs) and 32 x 1 (8-byte loads: the per-CU request rate, not the byte
-// count, limits a streaming workgroup). A forced split
-// (edsl_hip_set_gemv_ksplit) limits the choice to the widths that can take it.
-bool plan_gemv(const DeviceState& ds, int64_t M, int64_t N, int64_t K, bool realign, int* cols_out, int* ks_out) {
+// workgroup. For each, the K split is the one of least cost: the time of the
+// rounds of workgroups over the CUs, in units of a full chip, plus the bytes
+// of the partial sums (written and read once) over those of W. The first width
+// that keeps three quarters of the CUs busy is taken; when none does, the plan
+// with the most workgroups. Every wave keeps >= 2 steps of 16 rows. The order
+// is measured (M=16, K=N=8192 on MI355X): 128 columns x 4 splits beat 256 x 8
+// (more partial traffic), 64 x 2 (256-byte row runs) and 32 x 1 (8-byte loads:
+// the per-CU request rate, not the byte count, limits a streaming workgroup).
+// Splits need not be powers of two: 48x4096x4097 has 33 blocks of 128, and 8
+// splits put two workgroups on 8 of the CUs (40.3 us against 28.0 us for 7). A
+// forced split (edsl_hip_set_gemv_ksplit) limits the choice to the widths that
+// can take it.
+bool plan_gemv(const DeviceState& ds, int64_t M, int64_t N, int64_t K, int* cols_out, int* ks_out) {
   static const int kCols[] = {128, 256, 64, 32};
   if (N < 1 || K % 16 != 0) return false;
   int best_cols = 0, best_ks = 0;
   int64_t best_wgs = 0;
   // K is walked in 16-row chunks spread evenly over the ks x wk wave slices;
   // the automatic plan gives every slice at least two, a forced split at
-  // least one. Realigned rows leave the last row of W to the K tail, so K =
-  // 2^n falls one chunk short of the next split: there all slices but one
-  // get two.
-  const int64_t chunks = K / 16 + (realign ? 1 : 0);
+  // least one.
+  const int64_t chunks = K / 16;
   // Returns true when the width fills the chip.
   auto consider = [&](int cols) {
     if (g_force_cols > 0 && cols != g_force_cols) return false;
@@ -332,7 +334,16 @@ bool plan_gemv(const DeviceState& ds, int64_t M, int64_t N, int64_t K, bool real
       ks = g_force_ksplit;
     } else {
       if (chunks < 2 * wk) return false;
-      while (groups * ks < ds.cus && ks * 2 <= gemv_f32_max_ksplit() && chunks >= 2 * wk * ks * 2) ks *= 2;
+      double best = 0;
+      for (int s = 1; s <= gemv_f32_max_ksplit() && chunks >= 2 * wk * s; ++s) {
+        const int64_t rounds = (groups * s + ds.cus - 1) / ds.cus;
+        const double cost = (double)(rounds * ds.cus) / (double)(groups * s) +
+                            (s > 1 ? 2.0 * (double)s * (double)M / (double)K : 0.0);
+        if (s == 1 || cost < best) {
+          best = cost;
+          ks = s;
+        }
+      }
     }
     const int64_t wgs = groups * ks;
     if (wgs > best_wgs) {
@@ -340,14 +351,10 @@ bool plan_gemv(const DeviceState& ds, int64_t M, int64_t N, int64_t K, bool real
       best_ks = ks;
       best_wgs = wgs;
     }
-    return wgs >= ds.cus;
+    return 4 * wgs >= 3 * ds.cus;
   };
-  // Realigned rows (four columns per lane) stream at 1.5-2x the rate of the
-  // 4-byte loads that 32-column blocks fall back to: those are taken only when
-  // no wider block fits.
   for (int cols : kCols)
-    if ((!realign || cols > 32) && consider(cols)) break;
-  if (realign && best_cols == 0) consider(32);
+    if (consider(cols)) break;
   if (best_cols == 0) return false;
   *cols_out = best_cols;
   *ks_out = best_ks;
@@ -364,64 +371,38 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
   const int M = (int)L.M, N = (int)L.N, K = (int)L.K;
 
   // Small M: the streaming kernel walks the first K16 = K - K % 16 rows; the
-  // reduce kernel adds the rest. Operands need no alignment: X rows that are
-  // not 16-byte aligned are read with 4-byte loads; W rows that are not (or N
-  // not a multiple of 4) are realigned from 16-byte chunks or read per column,
-  // with Y and the bias written and read per element.
+  // reduce kernel adds the rest. Operands need no alignment.
   int gemv_cols = 0, gemv_ks = 0;
   const bool w_vec = al16(L.w) && al16(L.y) && (!bias_al || al16(bias_al)) && L.ldw % 4 == 0 &&
                      L.ldy % 4 == 0 && N % 4 == 0;
-  // Realigned W rows (two aligned 16-byte chunks per lane and row) leave the
-  // last row of W to the reduce kernel's K tail.
-  const bool w_realign = !w_vec && N >= 4;
-  const int K16 = w_realign ? ((K - 1) & ~15) : (K & ~15);
-  // With W, Y or the bias not vector-aligned the small-M kernel streams W
-  // realigned at ~3.3-4.4 TB/s with one row block (~2 TB/s with 4-byte loads:
-  // N < 4 or 32-column blocks); the 32x32 any-shape tile reads W once per 32
-  // rows of M at ~2.8 TB/s. Measured, small-M kernel vs tile: 16x8192x8191 61
-  // vs 134 us, 16x4096x50257 249 vs 290, 17x4096x50257 259 vs 283,
-  // 32x4096x50257 300 vs 292, 48x4096x50257 362 vs 495, 64x4096x50257 442 vs
-  // 498, 64x2048x50257 254 vs 258, 64x8192x8191 115 vs 166, 33x2048x4097 32
-  // vs 41; short K goes to the tile: 32x1024x32001 57 vs 49. So realigned
-  // rows take the small-M kernel for K >= 2048 (K >= 1024 with one row
-  // block), with at least 8 MiB of W: below that the layer is latency-bound
-  // and the tile's single launch wins (4x512x511: 8.4 vs 13.9 us;
-  // 16x1024x1023: even; 8x2048x2047 at 16 MiB: 15.6 vs 30.6). With 4-byte
-  // loads: when the plan splits K and M <= 48 (measured up to three row
-  // blocks). A forced split (edsl_hip_set_gemv_ksplit) or
-  // edsl_hip_set_small_m(1) takes the small-M kernel.
-  const bool gemv_planned =
-      M >= 1 && M <= kGemvMaxM && K16 > 0 && plan_gemv(ds, M, N, K16, w_realign, &gemv_cols, &gemv_ks);
-  const bool realigned_plan = w_realign && gemv_cols > 32;
+  const int K16 = K & ~15;
   const int row_blocks = (M + 15) / 16;
-  const bool w_large = (int64_t)K * N * (int64_t)sizeof(float) >= (8 << 20);
-  // Vector-aligned W: the small-M kernel's parallelism comes from splitting
-  // K, the tiles' from the M x N output, so short K favours the tiles (32x32
-  // tiles read W once up to 32 rows, twice up to 64). Measured on one box,
-  // small-M kernel vs 32x32 tile: one row block 16x512x512 5.7 vs 6.1 us,
-  // 16x256x4096 5.7 vs 4.4, 1x256x256 5.0 vs 4.2; two 32x1024x1024 7.9 vs
-  // 9.4, 32x512x512 7.5 vs 6.1; three 48x2048x2048 14.3 vs 16.9,
-  // 48x1024x4096 14.3 vs 10.4; four 64x8192x8192 101 vs 115, 64x4096x8192
-  // 52 vs 57, 64x2048x1024 11.2 vs 16.3, 64x2048x8192 32 vs 28, 64x2048x2048
-  // 17.4 vs 16.4, 64x1024x1024 10.3 vs 9.5. With X rows not 16-byte aligned
-  // the tiles are the any-shape ones and the small-M kernel is kept.
+  // The small-M kernel's parallelism comes from splitting K, the tiles' from
+  // the M x N output, so short K favours the tiles (32x32 tiles read W once up
+  // to 32 rows, twice up to 64). Measured on one box, small-M kernel vs 32x32
+  // tile: one row block 16x512x512 5.7 vs 6.1 us, 16x256x4096 5.7 vs 4.4,
+  // 1x256x256 5.0 vs 4.2; two 32x1024x1024 7.9 vs 9.4, 32x512x512 7.5 vs 6.1;
+  // three 48x2048x2048 14.3 vs 16.9, 48x1024x4096 14.3 vs 10.4; four
+  // 64x8192x8192 101 vs 115, 64x4096x8192 52 vs 57, 64x2048x1024 11.2 vs 16.3,
+  // 64x2048x8192 32 vs 28, 64x2048x2048 17.4 vs 16.4, 64x1024x1024 10.3 vs
+  // 9.5. Unaligned W costs the small-M kernel little, but the tiles are then
+  // the slower any-shape ones: one row block 16x400x7001 8.1 vs 10.7,
+  // 16x256x4095 6.2 vs 5.4; two 32x512x511 7.3 vs 8.7, 32x256x2047 6.4 vs 5.6;
+  // three and four 48x1024x1023 9.4 vs 16.9, 64x1024x1023 11.1 vs 16.9,
+  // 64x2048x2047 16.7 vs 31.5, 64x700x7001 23.9 vs 20.7, 33x384x1001 8.5 vs
+  // 8.1. With only X rows not 16-byte aligned the small-M kernel is kept. A
+  // forced split (edsl_hip_set_gemv_ksplit) or edsl_hip_set_small_m(1) takes
+  // the small-M kernel.
   const bool x_vec = al16(L.x) && L.ldx % 4 == 0;
-  bool vec_small_m = true;
-  if (x_vec) {
-    if (row_blocks == 1)
-      vec_small_m = K >= 512;
-    else if (row_blocks == 2)
-      vec_small_m = K >= 1024;
-    else if (row_blocks == 3)
-      vec_small_m = K >= 2048;
-    else
-      vec_small_m = K >= 4096 || (int64_t)K >= 2 * (int64_t)N;
-  }
-  if (gemv_planned &&
-      ((w_vec && vec_small_m) || g_force_ksplit > 0 || g_force_small_m == 1 ||
-       (realigned_plan && w_large && (K >= 2048 || (row_blocks == 1 && K >= 1024))) ||
-       (!w_vec && !realigned_plan && gemv_ks > 1 && M <= 48))) {
-    const bool x_ok = x_vec;
+  bool small_m = true;
+  if (!w_vec)
+    small_m = K >= (row_blocks == 1 ? 384 : row_blocks == 2 ? 512 : 1024);
+  else if (x_vec && row_blocks <= 3)
+    small_m = K >= 512 << (row_blocks - 1);
+  else if (x_vec)
+    small_m = K >= 4096 || (int64_t)K >= 2 * (int64_t)N;
+  small_m = small_m || g_force_ksplit > 0 || g_force_small_m == 1;
+  if (small_m && M >= 1 && M <= kGemvMaxM && K16 > 0 && plan_gemv(ds, M, N, K16, &gemv_cols, &gemv_ks)) {
     const bool tail = K16 < K;
     if (tail && gemv_ks == 1) gemv_ks = 2;  // the reduce kernel adds the tail
     GemvF32Args a{};
@@ -445,12 +426,7 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
     const bool scratch = a.ksplit > 1;
     const size_t part_bytes = scratch ? (size_t)a.ksplit * 16 * mb * a.ldp * sizeof(float) : 0;
     if (!has_bias) a.bias = nullptr;
-    // Two columns per lane (32-column blocks) read unaligned rows per column.
-    a.w_mode = w_vec ? kWVector : (realigned_plan ? kWRealign : kWScalar);
-    // Vector rows only where the operands allow them; the other modes are
-    // correct on any rows (a bias the epilogue does not add may still have
-    // ruled vector rows out, see DenseLaunch::plan_bias).
-    if (a.w_mode == kWVector && !gemv_f32_vector_rows(a)) fail(kErrInternal, "small-M W mode mismatch");
+    a.w_mode = gemv_f32_w_mode(a.W, a.ldw, N);
     if (fixed) {
       // Caller-fixed scratch: nothing is allocated and no cross-stream
       // ordering is added.
@@ -466,8 +442,8 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
     if (scratch && !fixed) scratch_end(ds, stream);
     set_plan("gemv_f32 mb=%d ksplit=%d cols=%d grid=%d%s%s%s%s%s", mb, a.ksplit, gemv_cols,
              ((N + gemv_cols - 1) / gemv_cols) * a.ksplit, a.ksplit > 1 ? " +reduce" : "",
-             x_ok ? "" : " +xunaligned",
-             a.w_mode == kWVector ? "" : a.w_mode == kWRealign ? " +wrealigned" : " +wunaligned", tail ? " +ktail" : "",
+             x_vec ? "" : " +xunaligned",
+             w_vec ? "" : N >= 4 && gemv_cols > 32 ? " +wrealigned" : " +wunaligned", tail ? " +ktail" : "",
              fixed && scratch ? " +fixed-scratch" : "");
     return;
   }

@@ -1,0 +1,44 @@
+"""The small-M kernel on W rows of any alignment, with K splits that are not
+powers of two (as many workgroups as fill the CUs once or twice)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from conftest import assert_f32_parity
+from mlir_edsl_hip import _native
+
+pytestmark = pytest.mark.gpu
+
+
+# W's rows start on 128-byte lines (streamed loads), on 16-byte ones, or on
+# neither (both cached, column blocks mapped by XCD: total workgroups that 8
+# does and does not divide); N that ends inside a lane's four columns, at its
+# end, or one column into a block.
+@pytest.mark.parametrize("M, K, N, pad, off", [
+    (16, 1040, 4096, 0, 0),    # 128-byte rows
+    (16, 1040, 4096, 4, 4),    # 16-byte rows
+    (16, 1040, 4097, 0, 0), (3, 1040, 4098, 0, 1), (20, 1040, 4099, 1, 3), (48, 1040, 4097, 0, 2),
+    (64, 1040, 8191, 0, 0), (33, 1029, 1000, 1, 0), (1, 1029, 5, 0, 0), (17, 1029, 3, 0, 0),
+])
+def test_rows_of_any_alignment(M, K, N, pad, off):
+    import torch
+    from mlir_edsl_hip.device import dense_launch
+    rng = np.random.default_rng(M + 3 * K + 7 * N + pad + off)
+    X = rng.standard_normal((M, K), dtype=np.float32)
+    W = (rng.standard_normal((K, N), dtype=np.float32) / np.float32(np.sqrt(K))).astype(np.float32)
+    b = rng.uniform(-0.1, 0.1, N).astype(np.float32)
+    buf = torch.full((K * (N + pad) + off,), float("nan"), device="cuda")
+    tW = buf[off:].view(K, N + pad)[:, :N]
+    tW.copy_(torch.from_numpy(W))
+    ybuf = torch.full((M * (N + pad) + off + 8,), 7.0, device="cuda")  # nothing past the rows is written
+    tY = ybuf[off:off + M * (N + pad)].view(M, N + pad)[:, :N]
+    dense_launch(torch.from_numpy(X).cuda(), tW, torch.from_numpy(b).cuda(), tY, _native.EPI_BIAS_RELU)
+    torch.cuda.synchronize()
+    assert _native.last_plan().startswith("gemv_f32"), _native.last_plan()
+    assert_f32_parity(tY.cpu().numpy(), oracle.dense_f32_chains(X, W, b, "relu"), K)
+    assert (ybuf[:off] == 7.0).all() and (ybuf[off + M * (N + pad):] == 7.0).all()
+    if pad:
+        gap = ybuf[off:off + M * (N + pad)].view(M, N + pad)[:, N:]
+        assert (gap == 7.0).all()
