@@ -61,6 +61,20 @@ __device__ __forceinline__ float apply_epilogue_f32(float acc, float b, float al
   return y;
 }
 
+// The epilogue by a code known at run time (uniform).
+__device__ __forceinline__ float epilogue_rt(float acc, float b, float alpha, int epi) {
+  switch (epi) {
+    case epi_code(false, ACT_NONE): return apply_epilogue_f32<epi_code(false, ACT_NONE)>(acc, b, alpha);
+    case epi_code(true, ACT_NONE): return apply_epilogue_f32<epi_code(true, ACT_NONE)>(acc, b, alpha);
+    case epi_code(false, ACT_RELU): return apply_epilogue_f32<epi_code(false, ACT_RELU)>(acc, b, alpha);
+    case epi_code(true, ACT_RELU): return apply_epilogue_f32<epi_code(true, ACT_RELU)>(acc, b, alpha);
+    case epi_code(false, ACT_LEAKY): return apply_epilogue_f32<epi_code(false, ACT_LEAKY)>(acc, b, alpha);
+    case epi_code(true, ACT_LEAKY): return apply_epilogue_f32<epi_code(true, ACT_LEAKY)>(acc, b, alpha);
+    case epi_code(false, ACT_IF_RELU): return apply_epilogue_f32<epi_code(false, ACT_IF_RELU)>(acc, b, alpha);
+    default: return apply_epilogue_f32<epi_code(true, ACT_IF_RELU)>(acc, b, alpha);
+  }
+}
+
 template <int EPI>
 __device__ __forceinline__ int32_t apply_epilogue_i32(int32_t acc, int32_t b) {
   // arith.addi wraps modulo 2^32.

@@ -55,19 +55,6 @@ constexpr int waves_per_wg(int mb, int wn) { return (mb == 1 ? 4 : 8) > wn ? (mb
 constexpr int kMaxSplit = 16;
 constexpr int kMaxTail = 16;  // rows of the K tail (GemvF32Args::k_end - K)
 
-__device__ __forceinline__ float epilogue_rt(float acc, float b, float alpha, int epi) {
-  switch (epi) {
-    case epi_code(false, ACT_NONE): return apply_epilogue_f32<epi_code(false, ACT_NONE)>(acc, b, alpha);
-    case epi_code(true, ACT_NONE): return apply_epilogue_f32<epi_code(true, ACT_NONE)>(acc, b, alpha);
-    case epi_code(false, ACT_RELU): return apply_epilogue_f32<epi_code(false, ACT_RELU)>(acc, b, alpha);
-    case epi_code(true, ACT_RELU): return apply_epilogue_f32<epi_code(true, ACT_RELU)>(acc, b, alpha);
-    case epi_code(false, ACT_LEAKY): return apply_epilogue_f32<epi_code(false, ACT_LEAKY)>(acc, b, alpha);
-    case epi_code(true, ACT_LEAKY): return apply_epilogue_f32<epi_code(true, ACT_LEAKY)>(acc, b, alpha);
-    case epi_code(false, ACT_IF_RELU): return apply_epilogue_f32<epi_code(false, ACT_IF_RELU)>(acc, b, alpha);
-    default: return apply_epilogue_f32<epi_code(true, ACT_IF_RELU)>(acc, b, alpha);
-  }
-}
-
 // WM (GemvF32Args::w_mode): kWVector and kWShared (N >= 4) -- a lane's CPL
 // columns are one vector load per row, whatever the alignment of W and its row
 // stride; a lane whose columns reach past N loads the last CPL columns instead

@@ -381,4 +381,22 @@ int plan_f32_tile(const F32TileQuery& q) {
   return cfg;
 }
 
+int plan_f32_small(const F32TileQuery& q, bool stream_rows) {
+  if (q.forced >= 0 || q.M < 1 || q.N < 1 || q.K < 1 || q.K > 1024) return 0;
+  const int64_t tiles = ((q.M + 15) / 16) * ((q.N + 15) / 16);
+  if (stream_rows) {
+    if (tiles > 2 * q.cus) return 0;
+  } else {
+    const int cfg = plan_f32_tile(q);
+    if (cfg == kF32T32 || cfg == kF32T32Edge) {
+      if (2 * tiles > 5 * q.cus) return 0;
+    } else if (gemm_f32_config(cfg).guard == kGuardScalar) {
+      if (2 * tiles > 9 * q.cus) return 0;
+    } else {
+      return 0;
+    }
+  }
+  return q.K <= 448 ? 4 : 8;
+}
+
 }  // namespace edsl

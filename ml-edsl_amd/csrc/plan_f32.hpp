@@ -81,6 +81,24 @@ struct F32TileQuery {
 // The configuration for a tiled fp32 layer (M, N, K >= 0).
 int plan_f32_tile(const F32TileQuery& q);
 
+// Waves per workgroup (4 or 8) of the 16x16 tiles for small outputs
+// (gemm_f32_small.hip), or 0 where the layer's other kernel is the better one:
+// the small-M streaming kernel (stream_rows), else the planned tile. Only for
+// K <= 1024 (16x2048x1024 6.9 us streamed, 6.9-8.5 us on 16x16 tiles). Same
+// box, us, against 16x16 tiles:
+//  * streamed rows, up to two 16x16 tiles per CU: 16x512x512 5.8 / 3.3,
+//    16x1024x4096 7.7 / 5.2, 64x512x256 9.9 / 3.4, 16x512x8192 7.6 / 5.1;
+//  * the LDS-staged 32x32 tiles, up to 2.5: 64x256x256 4.3 / 2.8, 256x1024x256
+//    9.4 / 5.0, 300x512x300 6.9 / 5.0, 400x256x400 4.9 / 4.4; with more
+//    they tie or lose (100x64x2000 4.0 / 4.1, 512x64x512 3.7 / 4.2);
+//  * the any-shape tiles, up to 4.5: 255x255x255 7.3 / 3.3, 401x511x399
+//    10.6 / 7.1, 513x1023x511 20.4 / 16.4;
+//  * the other tiles (32x32 R x C and larger) fill the chip and win:
+//    512x256x512 3.9 / 5.7; the exact 16x16 tile too: 128x128x128 2.4 / 2.5.
+// Eight waves from K = 449 on (16x512x4096 3.9 with four, 3.7 with eight;
+// 256x256x256 3.1 either way).
+int plan_f32_small(const F32TileQuery& q, bool stream_rows);
+
 // The one-wave tiles read A and B through buffer descriptors with 32-bit
 // byte offsets: 128 rows of A from a tile's first row, and all K rows of B
 // (plus a partial group's overrun) from a tile's first column, must be

@@ -401,6 +401,35 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
     small_m = K >= 512 << (row_blocks - 1);
   else if (x_vec)
     small_m = K >= 4096 || (int64_t)K >= 2 * (int64_t)N;
+  const F32TileQuery query{M, N, K, L.ldx, L.ldw, aligned, ds.cus, g_force_cfg};
+  GemmF32Args t{};  // the tiled kernels' arguments
+  t.A = static_cast<const float*>(L.x);
+  t.B = static_cast<const float*>(L.w);
+  t.bias = static_cast<const float*>(L.bias);
+  t.C = static_cast<float*>(L.y);
+  t.lda = L.ldx;
+  t.ldb = L.ldw;
+  t.ldc = L.ldy;
+  t.M = M;
+  t.N = N;
+  t.K = K;
+  t.alpha = L.alpha;
+
+  // Small outputs with short K: 16x16 tiles in one launch, no scratch.
+  const bool stream_rows = M >= 1 && M <= kGemvMaxM && small_m;
+  const bool tuned_small_m = g_force_ksplit > 0 || g_force_cols > 0 || g_force_small_m == 1;
+  const int waves = tuned_small_m ? 0 : plan_f32_small(query, stream_rows);
+  if (waves > 0) {
+    check_hip(launch_gemm_f32_small(waves, L.epi, t, stream), "gemm_f32_small launch");
+    const int grid = ((M + 15) / 16) * ((N + 15) / 16);
+    if (M <= kGemvMaxM && (small_m || !w_vec))
+      set_plan("gemv_f32 mb=%d ksplit=%d cols=16 tile=16x16 grid=%d%s%s%s", row_blocks, waves, grid,
+               x_vec ? "" : " +xunaligned", w_vec ? "" : " +wunaligned", K % 16 ? " +ktail" : "");
+    else
+      set_plan("gemm_f32 cfg=f32_16x16_anyshape_k%d grid=%d", waves, grid);
+    return;
+  }
+
   small_m = small_m || g_force_ksplit > 0 || g_force_small_m == 1;
   if (small_m && M >= 1 && M <= kGemvMaxM && K16 > 0 && plan_gemv(ds, M, N, K16, &gemv_cols, &gemv_ks)) {
     const bool tail = K16 < K;
@@ -449,24 +478,12 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
   }
 
   static_assert(kF32SmallM == kGemvMaxM, "the tile planner's small-M rule covers the small-M kernel's rows");
-  const int cfg = plan_f32_tile(F32TileQuery{M, N, K, L.ldx, L.ldw, aligned, ds.cus, g_force_cfg});
+  const int cfg = plan_f32_tile(query);
   const GemmF32Config& g = gemm_f32_config(cfg);
-  GemmF32Args a{};
-  a.A = static_cast<const float*>(L.x);
-  a.B = static_cast<const float*>(L.w);
-  a.bias = static_cast<const float*>(L.bias);
-  a.C = static_cast<float*>(L.y);
-  a.lda = L.ldx;
-  a.ldb = L.ldw;
-  a.ldc = L.ldy;
-  a.M = M;
-  a.N = N;
-  a.K = K;
-  a.alpha = L.alpha;
-  a.tiles_m = (M + g.bm - 1) / g.bm;
-  a.tiles_n = (N + g.bn - 1) / g.bn;
-  check_hip(launch_gemm_f32(cfg, L.epi, a, stream), "gemm_f32 launch");
-  set_plan("gemm_f32 cfg=%s grid=%d", g.name, a.tiles_m * a.tiles_n);
+  t.tiles_m = (M + g.bm - 1) / g.bm;
+  t.tiles_n = (N + g.bn - 1) / g.bn;
+  check_hip(launch_gemm_f32(cfg, L.epi, t, stream), "gemm_f32 launch");
+  set_plan("gemm_f32 cfg=%s grid=%d", g.name, t.tiles_m * t.tiles_n);
 }
 
 void launch_i32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream) {
