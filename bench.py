@@ -54,10 +54,13 @@ for _p in (ROOT, os.path.join(ROOT, "ml-edsl_amd")):
 METRIC = "fused matmul+bias+ReLU TFLOP/s & % roofline (4096^3 fp32); GB/s at M=16"
 PEAK = {  # MI355X published dense peaks
     "fp32_mfma_tflops": 157.3,
+    # fp32 layers as six exact bf16 products (gemm_f32_split.hip): a sixth of
+    # the dense bf16 rate bounds them
+    "bf16x6_mfma_tflops": round(2500.0 / 6, 1),
     "int8_mfma_tops": 5000.0,
     "hbm_gbs": 8000.0,
 }
-KERNEL_NAMES = {"c1": "gemm_f32_direct16_kernel", "c2": "gemm_f32_direct_rc_kernel", "c3": "gemm_f32_direct_kernel",
+KERNEL_NAMES = {"c1": "gemm_f32_direct16_kernel", "c2": "gemm_f32_direct_rc_kernel", "c3": "gemm_f32_split_kernel",
                 "c4": "gemv_f32_kernel + gemv_reduce_kernel", "c5": "narrow_i8_kernel + gemm_i8_ksplit_kernel",
                 "c3s8": "gemm_f32_direct64_kernel", "c4s8": "gemv_f32_kernel + gemv_reduce_kernel"}
 UNITS = {"c1": "TFLOP/s", "c2": "TFLOP/s", "c3": "TFLOP/s", "c4": "GB/s", "c5": "TOP/s",
@@ -348,9 +351,16 @@ def roofline_for(wname: str, r: dict, traffic: dict) -> dict:
                 "int8_mfma": {"achieved": round(tops, 2), "peak": PEAK["int8_mfma_tops"],
                               "unit": "TOP/s", "frac": round(tops / PEAK["int8_mfma_tops"], 4)}}
     achieved = w.flops / t / 1e12
-    return {"bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK["fp32_mfma_tflops"],
-            "unit": "TFLOP/s", "frac": round(achieved / PEAK["fp32_mfma_tflops"], 4), "traffic": tr,
-            "kernel": KERNEL_NAMES[wname], "algorithmic_flops": w.flops}
+    # Operations are the layer's 2 M N K, whichever matrix cores run them.
+    split = "split=bf16x6" in r["plan"]
+    peak = PEAK["bf16x6_mfma_tflops" if split else "fp32_mfma_tflops"]
+    out = {"bound": "mfma", "achieved": round(achieved, 2), "peak": peak,
+           "unit": "TFLOP/s", "frac": round(achieved / peak, 4), "traffic": tr,
+           "kernel": KERNEL_NAMES[wname], "algorithmic_flops": w.flops}
+    if split:
+        out["peak_is"] = ("dense bf16 MFMA / 6: every fp32 product as six bf16 products, fp32 error "
+                          f"(fp32 MFMA peak {PEAK['fp32_mfma_tflops']})")
+    return out
 
 
 # ------------------------------------------------------------ host buffers

@@ -97,6 +97,11 @@ __device__ float raw_buffer_load_f32(i32x4 rsrc, int voffset, int soffset, int a
 __device__ i32x4 raw_buffer_load_i32x4(i32x4 rsrc, int voffset, int soffset, int aux)
     __asm("llvm.amdgcn.raw.buffer.load.v4i32");
 
+// A store whose per-lane offset lies at or past the byte count is dropped.
+__device__ void raw_buffer_store_f32(float v, i32x4 rsrc, int voffset, int soffset, int aux)
+    __asm("llvm.amdgcn.raw.buffer.store.f32");
+constexpr int kAuxNonTemporal = 2;  // the gfx94x/gfx950 cache policy bit of the `aux` operand
+
 // Descriptor of `bytes` bytes from `base` (raw addressing: stride 0, the
 // 32-bit data format word of the gfx9 family), clamped to [0, 2^31 - 1].
 __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, int64_t bytes) {

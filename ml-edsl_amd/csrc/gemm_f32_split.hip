@@ -1,0 +1,418 @@
+// fp32 dense layer / matmul on the bf16 matrix cores, at fp32 precision, any
+// shape, row stride and alignment.
+//
+// C[M,N] = epilogue(A[M,K] x B[K,N] (+ bias[N])) -- the same op as the fp32
+// tiles (reference cpp/src/builders/LinalgBuilder.cpp:106-139, 180-239,
+// 301-339), for layers that fp32 MFMA bounds: its dense peak is 157 TFLOP/s,
+// that of bf16 MFMA 2500.
+//
+// Every fp32 value is split exactly into three bf16 values, x = h + m + l (h
+// the nearest bf16 of x, m that of x - h, l the rest: 8 + 8 + 8 significand
+// bits), and the product takes six of the nine bf16 products, each exact in
+// fp32: hh, hm, mh, mm, hl, lh. The three left out are below 2^-25 of a
+// product. They are summed in fp32 by v_mfma_f32_32x32x16_bf16, smallest
+// first. Relative 2-norm error against float64, N(0,1) data, K = 1024 / 2048 /
+// 4096: with one accumulator (TWO false) 4.6e-7 / 6.3e-7 / 1.05e-6, with the
+// five small products in one of their own (TWO true) 1.7e-7 / 2.7e-7 /
+// 3.8e-7; the fp32 MFMA chain 5.8e-7 / 8.0e-7 / 1.14e-6.
+//
+// Not every value splits exactly (the last remainder of a value below 2^-109
+// leaves bf16's range; h overflows within half a bf16 step of the largest
+// float), Inf - Inf is NaN, and a partial sum may overflow in one order and not
+// in another. A workgroup therefore ORs the low halves of all its last
+// remainders (zero exactly when they are bf16 values) and, at the end, tests
+// its sums; if any remainder was cut or any sum is not finite it recomputes its
+// tile on v_mfma_f32_16x16x4_f32 from the fp32 operands, with that path's
+// results for denormal, huge, infinite and NaN values.
+//
+// Bounds and layout. Splitting costs six VALU operations an element, so it is
+// done once per workgroup, on the way into LDS, never per wave: eight k of a
+// row of A (two 16-byte loads at any 4-byte alignment) or of a column of B
+// (eight 4-byte loads, 64 adjacent columns a wave) become one 16-byte piece of
+// each plane, stored in the order the MFMA reads (fragments of 32 rows x 16 k,
+// 1 KB, one 16-byte read per lane), rows XORed by the octet so that the eight
+// lanes of an LDS cycle never share banks (without it writes ran at a quarter
+// of the rate). The stages are double-buffered with one barrier per step; the
+// barrier stands before a step's last slice of MFMAs, whose operands are in
+// registers, so the next stage's first fragments are read behind those MFMAs.
+// Each octet's registers are reloaded with the step after next as soon as it
+// has been split, a full step ahead of its use (loading in one burst a slice
+// ahead cost 180 of 820 us at 4096^3). The K % BK rows are the first step, the
+// only masked one. Rows past M and columns past N read the last row or column;
+// their outputs are not stored.
+//
+// What bounds it is power: the full chip runs this loop at 1.7-1.8 GHz, a
+// register-only loop of the same MFMAs takes 491 us of the 612 us at 4096^3,
+// and without the LDS reads the loop would take 470 (256x128 tiles of eight
+// waves). Hence the 256x256 tile of four waves, each 128x128: half the LDS
+// reads per MFMA of 64x64 wave tiles. Measured, us, against the fp32 tiles:
+// 4096^3 612 / 900 (225 TFLOP/s), 4000x1024x4000 177 / 224; 2048^3 on eight
+// waves of 64x32 97 / 117 (four waves of 64x64: 102), 2001^3 101 / 153;
+// 10000x500x1000 on two workgroups of 128x128x16 per CU 82 / 93.
+#include "common.hpp"
+#include "kernels.hpp"
+
+#include <type_traits>
+
+namespace edsl {
+namespace {
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// Four floats at any 4-byte aligned address.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+constexpr int kPlanes = 3;
+
+__device__ __forceinline__ uint32_t cvt_pk_bf16(float a, float b) {
+  const bf16x2 p = __builtin_convertvector(f32x2{a, b}, bf16x2);
+  return __builtin_bit_cast(uint32_t, p);
+}
+__device__ __forceinline__ float bf_lo(uint32_t p) { return __builtin_bit_cast(float, p << 16); }
+__device__ __forceinline__ float bf_hi(uint32_t p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
+
+// Eight floats as three bf16 planes; ORs the bits of the last remainders into `lost`.
+__device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&p)[kPlanes], uint32_t& lost) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float a = x[2 * i], b = x[2 * i + 1];
+    const uint32_t h = cvt_pk_bf16(a, b);
+    const float ra = a - bf_lo(h), rb = b - bf_hi(h);
+    const uint32_t m = cvt_pk_bf16(ra, rb);
+    const float qa = ra - bf_lo(m), qb = rb - bf_hi(m);
+    p[0][i] = h;
+    p[1][i] = m;
+    p[2][i] = cvt_pk_bf16(qa, qb);
+    lost |= __builtin_bit_cast(uint32_t, qa) | __builtin_bit_cast(uint32_t, qb);
+  }
+}
+
+// BM x BN outputs per workgroup of WM x WN waves, BK-deep steps of K. TWO: the
+// small products in their own accumulator.
+template <int BM_, int BN_, int WM_, int WN_, int BK_, bool TWO_>
+struct SplitTile {
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, BK = BK_;
+  static constexpr bool TWO = TWO_;
+  static constexpr int kWaves = WM * WN;
+  static constexpr int kThreads = 64 * kWaves;
+  static constexpr int RB = BM / WM / 32, CB = BN / WN / 32;  // 32x32 blocks of a wave
+  static constexpr int KK = BK / 16;                          // MFMA steps of a stage
+  static constexpr int OPR = BK / 8;                          // octets per row
+  static constexpr int AO = BM * OPR / kThreads;              // octets a thread stages
+  static constexpr int BO = BN * OPR / kThreads;
+  static constexpr int kFrag = 1024;
+  static constexpr int kABytes = BM / 32 * KK * kPlanes * kFrag;
+  static constexpr int kBBytes = BN / 32 * KK * kPlanes * kFrag;
+  static constexpr int kStage = kABytes + kBBytes;
+  static constexpr int kLds = 2 * kStage;
+  static_assert(BM * OPR % kThreads == 0 && BN * OPR % kThreads == 0, "octets per thread");
+  static_assert(BN % 64 == 0 && BM % 32 == 0, "tile");
+};
+
+// A wave's outputs from row m0 and column n0 on, from the fp32 operands on
+// v_mfma_f32_16x16x4_f32: a workgroup whose values do not all split exactly,
+// or whose sums are not all finite, recomputes its tile here.
+// 64 rows at a time (128 x 128 accumulators at once would spill).
+template <class C, int EPI>
+__device__ __forceinline__ void fp32_wave_rows(const GemmF32Args& args, int m0, int n0) {
+  constexpr int R = 4, CC = 2 * C::CB;  // 16x16 blocks
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4, r16 = lane & 15;
+  const int M = args.M, N = args.N, K = args.K;
+  const float* pa[R];
+  int col[CC];
+#pragma unroll
+  for (int i = 0; i < R; ++i) pa[i] = args.A + (int64_t)min(m0 + 16 * i + r16, M - 1) * args.lda;
+#pragma unroll
+  for (int c = 0; c < CC; ++c) col[c] = min(n0 + 16 * c + r16, N - 1);
+  f32x4 acc[R][CC] = {};
+#pragma unroll 1
+  for (int k0 = 0; k0 < K; k0 += 4) {
+    const int k = k0 + g, kc = min(k, K - 1);
+    const float* pb = args.B + (int64_t)kc * args.ldb;
+    float a[R], b[CC];
+#pragma unroll
+    for (int i = 0; i < R; ++i) a[i] = pa[i][kc];
+#pragma unroll
+    for (int c = 0; c < CC; ++c) b[c] = pb[col[c]];
+#pragma unroll
+    for (int i = 0; i < R; ++i) a[i] = k < K ? a[i] : 0.0f;
+#pragma unroll
+    for (int c = 0; c < CC; ++c) b[c] = k < K ? b[c] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int c = 0; c < CC; ++c) acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[c], acc[i][c], 0, 0, 0);
+  }
+#pragma unroll
+  for (int c = 0; c < CC; ++c) {
+    const int n = n0 + 16 * c + r16;
+    if (n >= N) continue;
+    const float bv = epi_has_bias(EPI) ? args.bias[n] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + 16 * i + 4 * g + e;
+        if (m < M) args.C[(int64_t)m * args.ldc + n] = apply_epilogue_f32<EPI>(acc[i][c][e], bv, args.alpha);
+      }
+  }
+}
+
+template <class C, int EPI>
+__device__ __forceinline__ void fp32_wave_tile(const GemmF32Args& args, int m0, int n0) {
+  static_assert(C::RB % 2 == 0, "64-row pieces");
+#pragma unroll 1
+  for (int i = 0; i < C::RB / 2; ++i) fp32_wave_rows<C, EPI>(args, m0 + 64 * i, n0);
+}
+
+template <class C, int EPI>
+__global__ void __launch_bounds__(C::kThreads)
+gemm_f32_split_kernel(GemmF32Args args) {
+  constexpr int RB = C::RB, CB = C::CB, KK = C::KK;
+  __shared__ __align__(16) char smem[C::kLds];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / C::WN, wn = wave % C::WN;
+  int tm, tn;
+  tile_coords(blockIdx.x, args.tiles_m, args.tiles_n, tm, tn);
+  const int m0 = tm * C::BM, n0 = tn * C::BN;
+  const int M = args.M, N = args.N, K = args.K;
+
+  // Sources of the octets this thread stages.
+  const float* pa[C::AO];
+  int la[C::AO];
+#pragma unroll
+  for (int i = 0; i < C::AO; ++i) {
+    const int idx = threadIdx.x + i * C::kThreads;
+    const int row = idx / C::OPR, o = idx % C::OPR;
+    pa[i] = args.A + (int64_t)min(m0 + row, M - 1) * args.lda + 8 * o;
+    la[i] = ((row / 32) * KK + o / 2) * kPlanes * C::kFrag + ((o % 2) * 32 + (row % 32 ^ o * (8 / C::OPR))) * 16;
+  }
+  int cb[C::BO], ob[C::BO], lb[C::BO];
+#pragma unroll
+  for (int i = 0; i < C::BO; ++i) {
+    const int idx = wave + i * C::kWaves;
+    const int c64 = idx % (C::BN / 64);
+    ob[i] = idx / (C::BN / 64);
+    const int col = c64 * 64 + lane;
+    cb[i] = min(n0 + col, N - 1);
+    lb[i] = C::kABytes + ((col / 32) * KK + ob[i] / 2) * kPlanes * C::kFrag +
+            ((ob[i] % 2) * 32 + (col % 32 ^ ob[i] * (8 / C::OPR))) * 16;
+  }
+
+  constexpr int kOct = C::AO + C::BO;
+  float raw[kOct][8];
+  auto load_octet = [&](int o, int k0) __attribute__((always_inline)) {
+    if (o < C::AO) {
+      const float* p = pa[o] + k0;
+      const f32x4u v0 = *reinterpret_cast<const f32x4u*>(p), v1 = *reinterpret_cast<const f32x4u*>(p + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        raw[o][e] = v0[e];
+        raw[o][4 + e] = v1[e];
+      }
+    } else {
+      const int i = o - C::AO;
+      const float* p = args.B + (int64_t)(k0 + 8 * ob[i]) * args.ldb;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) raw[o][e] = (p + e * args.ldb)[cb[i]];
+    }
+  };
+  auto load_tail = [&](int o, int k0) {
+    const int ko = o < C::AO ? 8 * (((int)threadIdx.x + o * C::kThreads) % C::OPR) : 8 * ob[o < C::AO ? 0 : o - C::AO];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int k = k0 + ko + e, kc = min(k, K - 1);
+      const float v = o < C::AO ? pa[o < C::AO ? o : 0][kc - ko] : (args.B + (int64_t)kc * args.ldb)[cb[o < C::AO ? 0 : o - C::AO]];
+      raw[o][e] = k < K ? v : 0.0f;
+    }
+  };
+  uint32_t lost = 0;
+  auto stage_octet = [&](char* st, int o) __attribute__((always_inline)) {
+    u32x4 p[kPlanes];
+    split8(raw[o], p, lost);
+    const int at = o < C::AO ? la[o] : lb[o - C::AO];
+#pragma unroll
+    for (int q = 0; q < kPlanes; ++q) *reinterpret_cast<u32x4*>(st + at + q * C::kFrag) = p[q];
+  };
+
+  f32x16 acc[RB][CB] = {};
+  f32x16 low[C::TWO ? RB : 1][C::TWO ? CB : 1] = {};
+  // Steps: the K % BK rows first, if any, then the full steps.
+  const int full = K / C::BK;
+  const int has_tail = K % C::BK != 0;
+  const int nit = full + has_tail;
+  auto k_of = [&](int it) { return (min(it, nit - 1) - has_tail) * C::BK; };  // full steps
+  if (has_tail) {
+#pragma unroll
+    for (int o = 0; o < kOct; ++o) load_tail(o, full * C::BK);
+  } else {
+#pragma unroll
+    for (int o = 0; o < kOct; ++o) load_octet(o, 0);
+  }
+#pragma unroll
+  for (int o = 0; o < kOct; ++o) stage_octet(smem, o);
+  if (nit > 1) {
+#pragma unroll
+    for (int o = 0; o < kOct; ++o) load_octet(o, k_of(1));
+  }
+  __syncthreads();
+
+  constexpr int BS = KK == 1 ? 2 : KK;  // sets of B fragments
+  bf16x8 a[2][kPlanes], b[BS][CB][kPlanes];
+  const int oa = wm * RB * KK * kPlanes * C::kFrag;
+  const int ob_ = C::kABytes + wn * CB * KK * kPlanes * C::kFrag;
+  int lofs[KK];
+#pragma unroll
+  for (int kk = 0; kk < KK; ++kk)
+    lofs[kk] = ((lane & 32) + (lane % 32 ^ (2 * kk + (lane >> 5)) * (8 / C::OPR))) * 16;
+  auto read_a = [&](const char* st, int slice, int set) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < kPlanes; ++q)
+      a[set][q] = *reinterpret_cast<const bf16x8*>(st + oa + lofs[slice % KK] + (slice * kPlanes + q) * C::kFrag);
+  };
+  auto read_b = [&](const char* st, int kk, int set) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < CB; ++j)
+#pragma unroll
+      for (int q = 0; q < kPlanes; ++q)
+        b[set][j][q] = *reinterpret_cast<const bf16x8*>(st + ob_ + lofs[kk] + ((j * KK + kk) * kPlanes + q) * C::kFrag);
+  };
+  constexpr int kSlices = RB * KK;
+  static_assert(kSlices % 2 == 0, "A sets alternate by slice");
+  read_a(smem, 0, 0);
+  read_b(smem, 0, 0);
+  auto step = [&](int it, auto set_c) __attribute__((always_inline)) {
+    constexpr int S = decltype(set_c)::value;  // parity of the step
+    const char* st = smem + S * C::kStage;
+    char* sn = smem + (S ^ 1) * C::kStage;
+    const int k2 = k_of(it + 2);
+#pragma unroll
+    for (int sl = 0; sl < kSlices; ++sl) {
+      const int i = sl / KK, kk = sl % KK;
+      const int bs = KK == 1 ? S : kk;
+      if (sl == kSlices - 1) {
+        __syncthreads();
+        read_a(sn, 0, (sl + 1) & 1);
+        read_b(sn, 0, KK == 1 ? S ^ 1 : 0);
+      } else {
+        read_a(st, sl + 1, (sl + 1) & 1);
+        if (i == 0 && kk + 1 < KK) read_b(st, kk + 1, kk + 1);
+      }
+      // Smallest products first.
+      constexpr int pa_[6] = {2, 0, 1, 1, 0, 0}, pb_[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+      for (int s = 0; s < 6; ++s)
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+          f32x16& t = C::TWO && s < 5 ? low[C::TWO ? i : 0][C::TWO ? j : 0] : acc[i][j];
+          t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[sl & 1][pa_[s]], b[bs][j][pb_[s]], t, 0, 0, 0);
+        }
+      if (sl < kSlices - 1) {
+        // Octets sl, sl + (kSlices - 1), ... of the next stage; each one's
+        // registers are then free for the octet of the step after.
+#pragma unroll
+        for (int o = sl; o < kOct; o += kSlices - 1) {
+          stage_octet(sn, o);
+          load_octet(o, k2);
+        }
+      }
+      // One MFMA, at most one LDS read, five VALU operations, and so on: the
+      // compiler otherwise puts the splitting after the MFMAs.
+      constexpr int kReads[2] = {3, 3 + 3 * CB};
+      const int reads = kReads[sl == kSlices - 1 || (i == 0 && kk + 1 < KK)];
+#pragma unroll
+      for (int m = 0; m < 6 * CB; ++m) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (m < reads) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  int it = 0;
+  for (; it + 1 < nit; it += 2) {
+    step(it, std::integral_constant<int, 0>{});
+    step(it + 1, std::integral_constant<int, 1>{});
+  }
+  if (it < nit) step(it, std::integral_constant<int, 0>{});
+
+  if constexpr (C::TWO)
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int j = 0; j < CB; ++j) acc[i][j] += low[i][j];
+  bool bad = (lost & 0xffffu) != 0;
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int j = 0; j < CB; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) bad |= !(__builtin_fabsf(acc[i][j][e]) < __builtin_huge_valf());
+  if (__syncthreads_or(bad)) {  // uniform
+    fp32_wave_tile<C, EPI>(args, m0 + wm * RB * 32, n0 + wn * CB * 32);
+    return;
+  }
+  // Lane: rows 8 (r/4) + 4 (lane/32) + r%4 and column lane%32 of a block, so
+  // each store writes two 128-byte row segments. The stores go through a
+  // descriptor of C's rows m0 .. M-1, whose range check drops rows past M;
+  // columns past N are sent out of range. (A branch per store cost an edge
+  // tile 20 us; ldc is below 2^21, so a tile's offsets fit 31 bits.)
+  const int half = lane >> 5, l32 = lane & 31;
+  const int ldc = (int)args.ldc;
+  const i32x4 rsrc = buffer_rsrc(args.C + (int64_t)m0 * ldc, (int64_t)(M - m0) * ldc * 4);
+#pragma unroll
+  for (int j = 0; j < CB; ++j) {
+    const int col = n0 + (wn * CB + j) * 32 + l32;
+    const float bv = epi_has_bias(EPI) && col < N ? args.bias[col] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+      const int at = (((wm * RB + i) * 32 + 4 * half) * ldc + col) * 4;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int dr = 8 * (r >> 2) + (r & 3);
+        raw_buffer_store_f32(apply_epilogue_f32<EPI>(acc[i][j][r], bv, args.alpha), rsrc,
+                             col < N ? at + dr * ldc * 4 : 0x7fffffff, 0, kAuxNonTemporal);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
+template <class C>
+hipError_t launch_tile(int epi, GemmF32Args a, hipStream_t stream) {
+  a.tiles_m = (a.M + C::BM - 1) / C::BM;
+  a.tiles_n = (a.N + C::BN - 1) / C::BN;
+  const dim3 grid(a.tiles_m * a.tiles_n), block(C::kThreads);
+#define EDSL_SPLIT_CASE(E) \
+  case E: hipLaunchKernelGGL((gemm_f32_split_kernel<C, E>), grid, block, 0, stream, a); break;
+  switch (epi) {
+    EDSL_SPLIT_CASE(epi_code(false, ACT_NONE))
+    EDSL_SPLIT_CASE(epi_code(true, ACT_NONE))
+    EDSL_SPLIT_CASE(epi_code(false, ACT_RELU))
+    EDSL_SPLIT_CASE(epi_code(true, ACT_RELU))
+    EDSL_SPLIT_CASE(epi_code(false, ACT_LEAKY))
+    EDSL_SPLIT_CASE(epi_code(true, ACT_LEAKY))
+    EDSL_SPLIT_CASE(epi_code(false, ACT_IF_RELU))
+    EDSL_SPLIT_CASE(epi_code(true, ACT_IF_RELU))
+    default: return hipErrorInvalidValue;
+  }
+#undef EDSL_SPLIT_CASE
+  return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_gemm_f32_split(int tile, int epi, GemmF32Args a, hipStream_t stream) {
+  if (a.M < 1 || a.N < 1 || a.K < 32 || a.ldc >= kF32SplitMaxLdc) return hipErrorInvalidValue;  // a full step of K
+  switch (tile) {
+    case kSplit256: return launch_tile<SplitTile<256, 256, 2, 2, 16, false>>(epi, a, stream);
+    case kSplit128W8: return launch_tile<SplitTile<128, 128, 2, 4, 32, true>>(epi, a, stream);
+    case kSplit128Pair: return launch_tile<SplitTile<128, 128, 2, 2, 16, false>>(epi, a, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace edsl

@@ -77,6 +77,7 @@ struct F32TileQuery {
   bool aligned;
   int cus;      // compute units of the device
   int forced;   // a configuration to take when it fits these operands, or -1
+  int64_t ldc = 0;  // row stride of C, in elements
 };
 // The configuration for a tiled fp32 layer (M, N, K >= 0).
 int plan_f32_tile(const F32TileQuery& q);
@@ -104,5 +105,19 @@ int plan_f32_small(const F32TileQuery& q, bool stream_rows);
 // (plus a partial group's overrun) from a tile's first column, must be
 // addressable that way.
 bool gemm_f32_direct_offsets_fit(int64_t K, int64_t lda, int64_t ldb);
+
+// The tiles on bf16 matrix cores at fp32 precision (gemm_f32_split.hip).
+enum F32SplitTile : int {
+  kSplitNone = -1,
+  kSplit256 = 0,   // 256x256x16, four waves, one workgroup per CU, one accumulator
+  kSplit128W8,     // 128x128x32, eight waves, one workgroup per CU, two accumulators
+  kSplit128Pair,   // 128x128x16, four waves, two workgroups per CU, one accumulator
+};
+// The split tile for a layer whose fp32 tile is `cfg` (plan_f32_tile), or
+// kSplitNone where the fp32 tile is the better one.
+int plan_f32_split(const F32TileQuery& q, int cfg);
+constexpr int64_t kF32SplitMaxLdc = 1 << 21;  // 256 rows of C within 31-bit byte offsets
+const char* f32_split_name(int tile);
+int64_t f32_split_grid(int tile, int64_t M, int64_t N);
 
 }  // namespace edsl

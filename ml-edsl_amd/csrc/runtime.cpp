@@ -401,7 +401,7 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
     small_m = K >= 512 << (row_blocks - 1);
   else if (x_vec)
     small_m = K >= 4096 || (int64_t)K >= 2 * (int64_t)N;
-  const F32TileQuery query{M, N, K, L.ldx, L.ldw, aligned, ds.cus, g_force_cfg};
+  const F32TileQuery query{M, N, K, L.ldx, L.ldw, aligned, ds.cus, g_force_cfg, L.ldy};
   GemmF32Args t{};  // the tiled kernels' arguments
   t.A = static_cast<const float*>(L.x);
   t.B = static_cast<const float*>(L.w);
@@ -482,6 +482,15 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
   const GemmF32Config& g = gemm_f32_config(cfg);
   t.tiles_m = (M + g.bm - 1) / g.bm;
   t.tiles_n = (N + g.bn - 1) / g.bn;
+  // Layers that fp32 MFMA bounds run on the bf16 matrix cores, at fp32
+  // precision, in place of their fp32 tile.
+  const int split = plan_f32_split(query, cfg);
+  if (split != kSplitNone) {
+    check_hip(launch_gemm_f32_split(split, L.epi, t, stream), "gemm_f32_split launch");
+    set_plan("gemm_f32 split=bf16x6 tile=%s grid=%lld in place of cfg=%s grid=%d", f32_split_name(split),
+             (long long)f32_split_grid(split, M, N), g.name, t.tiles_m * t.tiles_n);
+    return;
+  }
   check_hip(launch_gemm_f32(cfg, L.epi, t, stream), "gemm_f32 launch");
   set_plan("gemm_f32 cfg=%s grid=%d", g.name, t.tiles_m * t.tiles_n);
 }

@@ -1,0 +1,128 @@
+"""fp32 layers on the bf16 matrix cores (gemm_f32_split.hip): the three tiles
+at sizes that divide and do not divide them (M, N and K remainders, rows off
+16-byte alignment, NaN in every padding element), every epilogue, and the
+values that do not split exactly -- denormal, near the largest float, infinite,
+NaN -- which the tile that holds them recomputes on fp32 MFMA."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from conftest import assert_f32_parity
+from mlir_edsl_hip import _native
+
+pytestmark = pytest.mark.gpu
+
+# (M, K, N): the split tile the planner takes
+SHAPES = [((3840, 512, 3840), "256x256x16"), ((4000, 271, 4001), "256x256x16"),
+          ((2048, 1024, 2048), "128x128x32_w8"), ((2001, 543, 2003), "128x128x32_w8"),
+          ((2500, 1024, 2500), "128x128x16"), ((2500, 1030, 2496), "128x128x16")]
+
+_EPIS = [(_native.EPI_NONE, False, "none"), (_native.EPI_BIAS, True, "none"), (_native.EPI_RELU, False, "relu"),
+         (_native.EPI_BIAS_RELU, True, "relu"), (_native.EPI_LEAKY, False, "leaky"),
+         (_native.EPI_BIAS_LEAKY, True, "leaky"), (_native.EPI_IF_RELU, False, "if_relu"),
+         (_native.EPI_BIAS_IF_RELU, True, "if_relu")]
+
+
+def _inputs(M, K, N, seed):
+    rng = np.random.default_rng(seed)
+    X = rng.standard_normal((M, K), dtype=np.float32)
+    W = (rng.standard_normal((K, N), dtype=np.float32) / np.float32(np.sqrt(K))).astype(np.float32)
+    return X, W, rng.uniform(-0.1, 0.1, N).astype(np.float32)
+
+
+def _view(torch, a, pad, off, fill):
+    rows, cols = a.shape
+    buf = torch.full(((rows + 1) * (cols + pad) + off,), fill, device="cuda")
+    v = buf[off:off + rows * (cols + pad)].view(rows, cols + pad)[:, :cols]
+    v.copy_(torch.from_numpy(a))
+    return v, buf
+
+
+@pytest.mark.parametrize("shape, tile", SHAPES, ids=["x".join(map(str, s)) for s, _ in SHAPES])
+def test_split_tiles(shape, tile):
+    import torch
+    from mlir_edsl_hip.device import dense_launch
+    M, K, N = shape
+    X, W, b = _inputs(M, K, N, M + K + N)
+    tb = torch.from_numpy(b).cuda()
+    ref = oracle.dense_f32_chains(X, W, b, "relu")
+    for pad, off in ((0, 0), (3, 1)):
+        tX, tW = (_view(torch, a, pad, off, float("nan"))[0] for a in (X, W))
+        tY, ybuf = _view(torch, np.full((M, N), 5.0, np.float32), pad, off, 7.0)
+        dense_launch(tX, tW, tb, tY, _native.EPI_BIAS_RELU)
+        torch.cuda.synchronize()
+        if pad == 0:
+            assert f"split=bf16x6 tile={tile} " in _native.last_plan(), _native.last_plan()
+        got = tY.cpu().numpy()
+        assert_f32_parity(got, ref, K)
+        tY.fill_(7.0)
+        assert (ybuf == 7.0).all()  # nothing else was written
+    # No larger error than the fp32 MFMA tile it replaces.
+    exact = torch.relu(tX.double() @ tW.double() + tb.double()).cpu().numpy()
+    norm = np.linalg.norm(exact)
+    err = np.linalg.norm(got - exact) / norm
+    assert err <= 2.5e-7 * np.sqrt(K / 256), err  # one fp32 chain: 2.9e-7 at K = 256, growing with sqrt(K)
+
+
+@pytest.mark.parametrize("epi, has_bias, act", _EPIS)
+def test_split_epilogues(epi, has_bias, act):
+    import torch
+    from mlir_edsl_hip.device import dense_launch
+    M, K, N = 2001, 512, 2003
+    X, W, b = _inputs(M, K, N, epi)
+    X[5] = 0.0  # sums of +0: -0 in the bias column gives +0
+    b[7], b[8] = -0.0, np.nan
+    tX, tW, tb = (torch.from_numpy(a).cuda() for a in (X, W, b))
+    Y = torch.full((M, N), 7.0, device="cuda")
+    dense_launch(tX, tW, tb if has_bias else None, Y, epi, 0.125)
+    torch.cuda.synchronize()
+    assert "split=bf16x6" in _native.last_plan()
+    got = Y.cpu().numpy()
+    assert_f32_parity(got, oracle.dense_f32_chains(X, W, b if has_bias else None, act, 0.125), K)
+    assert not np.signbit(got[5][got[5] == 0]).any()
+
+
+@pytest.mark.parametrize("M, K, N", [(3840, 512, 3840), (2001, 543, 2003), (2500, 1024, 2500)],
+                         ids=["256x256", "128x128_w8", "128x128"])
+def test_values_that_do_not_split(M, K, N):
+    """Denormal, huge, infinite and NaN operands give what the fp32 tiles
+    give; the tiles that hold none of them keep their bits."""
+    import torch
+    from mlir_edsl_hip.device import dense_launch, set_f32_config
+    X, W, b = _inputs(M, K, N, 3 * M + K)
+    tX, tW, tb = (torch.from_numpy(a).cuda() for a in (X, W, b))
+
+    def run(x, w, cfg=-1):
+        y = torch.full((M, N), 7.0, device="cuda")
+        set_f32_config(cfg)
+        try:
+            dense_launch(x, w, tb, y, _native.EPI_BIAS)
+            torch.cuda.synchronize()
+        finally:
+            set_f32_config(-1)
+        assert ("split=bf16x6" in _native.last_plan()) == (cfg < 0)
+        return y
+
+    anyshape = _native.f32_config_names().index("f32_128x128x32_mfma16_anyshape")
+    clean = run(tX, tW)
+    for value in (1e-40, -3.0e-38 / 2**12, 3.4e38, float("inf"), float("nan")):
+        x, w = tX.clone(), tW.clone()
+        x[M - 1, K - 1] = value
+        w[1, 3] = value
+        got, want = run(x, w), run(x, w, anyshape)
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+        ok = torch.isfinite(want)
+        # both sum the same fp32 products; 1e-4 sqrt(K) is the parity bar at unit scale
+        scale = want.abs().clamp_min(1.0)
+        assert (((got - want).abs() / scale)[ok] <= 1e-4 * K**0.5).all()
+        # Tiles of other rows and columns are untouched: 256 rows and columns from the edges.
+        assert torch.equal(got[:M - 512, 512:], clean[:M - 512, 512:])
+    # Operands that are tiny throughout lose nothing that fp32 keeps.
+    x = tX * 2.0**-118
+    got, ref = run(x, tW) - tb, x.double() @ tW.double()
+    y = torch.empty_like(got)
+    dense_launch(x, tW, None, y, _native.EPI_NONE)
+    torch.cuda.synchronize()
+    assert ((y.double() - ref).norm() / ref.norm()).item() <= 1e-5
