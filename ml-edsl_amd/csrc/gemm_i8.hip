@@ -16,7 +16,7 @@
 // the digit products X_i W_j with i + j <= 3, each such an int8 product,
 // shifted by 8 (i + j). Only the pairs that the values need are run: a layer
 // whose X holds 16-bit activations and whose W is int8 costs two int8 products
-// (512x1024x512: 12.9 us, 28.5 us with full 32-bit values on both sides; the
+// (512x1024x512: 11.8 us, 26.1 us with full 32-bit values on both sides; the
 // wrapping i32 product on the vector ALUs that this replaced: 405 us; 2048^3:
 // 40.6 and 133 us against 1169 us).
 //
@@ -189,14 +189,15 @@ __device__ __forceinline__ bool tile_is_wide(const GemmI32Args& a, int m0, int n
 // the 64-k chunks first, first + stride, ...: with X = sum_i 256^i X_i and W =
 // sum_j 256^j W_j in signed base-256 digits,
 //   X W mod 2^32 = sum over i + j <= 3 of 256^(i+j) X_i W_j,
-// each X_i W_j an exact int8 product (|sum| <= 2^14 K < 2^31). The pairs are
-// taken by falling i + j, the running total shifted up by 8 between them
-// (Horner), so one accumulator and one total suffice; adds wrap as arith.addi
-// does. Counts hold one byte per 64x64 tile: the wave runs the pairs that
-// any of its chunks needs, and reads a plane that a chunk does not have (never
-// written) as zeros through an out-of-range buffer offset, as it does chunks
-// past the last. Lane l of a counts register holds the count of the wave's
-// chunk 64 * (t / 64) + l, read back by lane number.
+// each X_i W_j an exact int8 product (|sum| <= 2^14 K < 2^31) that is shifted
+// and added to the total; adds wrap as arith.addi does. X_0 W_0 comes first:
+// every chunk has those planes, so it runs before the counts are looked at
+// (their loads are issued first; looked at first they cost a 512x1024x512
+// layer 1 us). Counts hold one byte per 64x64 tile: the wave then runs the
+// pairs that any of its chunks needs, and reads a plane that a chunk does not
+// have (never written) as zeros through an out-of-range buffer offset, as it
+// does chunks past the last. Lane l of a counts register holds the count of
+// the wave's chunk 64 * (t / 64) + l, read back by lane number.
 constexpr int kOutOfRange = 0x7fffffff;
 
 template <int D>
@@ -215,88 +216,91 @@ __device__ __forceinline__ void digits_wave(const GemmI32Args& a, int m0, int n0
 #pragma unroll
       for (int r = 0; r < 16; ++r) total[i][j][r] = 0;
   if (n <= 0) return;  // fewer chunks than waves
-  int dx = 1, dw = 1;
-  for (int t = lane; t < n; t += 64) {
-    dx = max(dx, (int)fx[(int64_t)t * stride]);
-    dw = max(dw, (int)fw[(int64_t)t * stride]);
-  }
-#pragma unroll
-  for (int d = 2; d <= kI8Digits; ++d) {  // wave maxima, uniform
-    if (__any(dx >= d)) dx = max(dx, d);
-    if (__any(dw >= d)) dw = max(dw, d);
-  }
-  dx = __builtin_amdgcn_readfirstlane(dx);
-  dw = __builtin_amdgcn_readfirstlane(dw);
+  const int u0 = min(lane, n - 1);
+  int cx = fx[(int64_t)u0 * stride], cw = fw[(int64_t)u0 * stride];  // counts of chunks 0 .. 63
 
   struct Chunk {
     i32x4 a[2][2], b[2][2];  // [32-k step][32-row block]
   };
-  for (int s = min(dx + dw - 2, kI8Digits - 1); s >= 0; --s) {
+  // total += 256^(di + dj) X_di W_dj; `all`: planes that every chunk has.
+  auto product = [&](int di, int dj, auto all) __attribute__((always_inline)) {
+    constexpr bool kAll = decltype(all)::value;
+    const i32x4 rsrc_a = buffer_rsrc(
+        a.A8p + (int64_t)di * a.plane_x + (int64_t)(m0 >> 5) * block_bytes, 2 * (int64_t)block_bytes);
+    const i32x4 rsrc_b = buffer_rsrc(
+        a.B8p + (int64_t)dj * a.plane_w + (int64_t)(n0 >> 5) * block_bytes, 2 * (int64_t)block_bytes);
+    int px = cx, pw = cw;
+    auto load = [&](Chunk& f, int t) __attribute__((always_inline)) {
+      const bool in = t < n;
+      int oa = in ? lane * 16 : kOutOfRange, ob = oa;
+      if constexpr (!kAll) {
+        if ((t & 63) == 0 && t > 0) {  // uniform: the counts of the next 64 chunks
+          const int u = min(t + lane, n - 1);
+          px = fx[(int64_t)u * stride];
+          pw = fw[(int64_t)u * stride];
+        }
+        if (__builtin_amdgcn_readlane(px, t & 63) <= di) oa = kOutOfRange;
+        if (__builtin_amdgcn_readlane(pw, t & 63) <= dj) ob = kOutOfRange;
+      }
+      const int at = (first + t * stride) * 2048;  // the chunk's two fragments of a block
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          f.a[k][i] = raw_buffer_load_i32x4(rsrc_a, oa, in ? at + k * 1024 + i * block_bytes : 0, 0);
+          f.b[k][i] = raw_buffer_load_i32x4(rsrc_b, ob, in ? at + k * 1024 + i * block_bytes : 0, 0);
+        }
+    };
+    i32x16 acc[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) total[i][j][r] = (int32_t)((uint32_t)total[i][j][r] << 8);
-    for (int di = max(0, s - dw + 1); di <= min(s, dx - 1); ++di) {
-      const int dj = s - di;
-      const i32x4 rsrc_a = buffer_rsrc(
-          a.A8p + (int64_t)di * a.plane_x + (int64_t)(m0 >> 5) * block_bytes, 2 * (int64_t)block_bytes);
-      const i32x4 rsrc_b = buffer_rsrc(
-          a.B8p + (int64_t)dj * a.plane_w + (int64_t)(n0 >> 5) * block_bytes, 2 * (int64_t)block_bytes);
-      int cx = 0, cw = 0;
-      auto load = [&](Chunk& f, int t) __attribute__((always_inline)) {
-        if ((t & 63) == 0) {  // uniform: the counts of the next 64 chunks
-          const int u = min(t + lane, n - 1);
-          cx = fx[(int64_t)u * stride];
-          cw = fw[(int64_t)u * stride];
-        }
-        const bool in = t < n;
-        const int at = (first + t * stride) * 2048;  // the chunk's two fragments of a block
-        const int oa = in && __builtin_amdgcn_readlane(cx, t & 63) > di ? lane * 16 : kOutOfRange;
-        const int ob = in && __builtin_amdgcn_readlane(cw, t & 63) > dj ? lane * 16 : kOutOfRange;
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+    Chunk f[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(f[d], d);
+#pragma unroll 1
+    for (int t = 0; t < n; t += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
 #pragma unroll
         for (int k = 0; k < 2; ++k)
 #pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            f.a[k][i] = raw_buffer_load_i32x4(rsrc_a, oa, in ? at + k * 1024 + i * block_bytes : 0, 0);
-            f.b[k][i] = raw_buffer_load_i32x4(rsrc_b, ob, in ? at + k * 1024 + i * block_bytes : 0, 0);
-          }
-      };
-      i32x16 acc[2][2];
+          for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
-      Chunk f[D];
-#pragma unroll
-      for (int d = 0; d < D; ++d) load(f[d], d);
-#pragma unroll 1
-      for (int t = 0; t < n; t += D) {
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-#pragma unroll
-          for (int k = 0; k < 2; ++k)
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-              for (int j = 0; j < 2; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f[d].a[k][i], f[d].b[k][j], acc[i][j], 0, 0, 0);
-          __builtin_amdgcn_sched_barrier(0);
-          load(f[d], t + d + D);
-          __builtin_amdgcn_sched_barrier(0);
-        }
+            for (int j = 0; j < 2; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f[d].a[k][i], f[d].b[k][j], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        load(f[d], t + d + D);
+        __builtin_amdgcn_sched_barrier(0);
       }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) total[i][j][r] = (int32_t)((uint32_t)total[i][j][r] + (uint32_t)acc[i][j][r]);
     }
+    const int shift = 8 * (di + dj);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          total[i][j][r] = (int32_t)((uint32_t)total[i][j][r] + ((uint32_t)acc[i][j][r] << shift));
+  };
+  product(0, 0, std::true_type{});
+  int dx = cx, dw = cw;
+  for (int t = lane + 64; t < n; t += 64) {
+    dx = max(dx, (int)fx[(int64_t)t * stride]);
+    dw = max(dw, (int)fw[(int64_t)t * stride]);
   }
+#pragma unroll
+  for (int d = kI8Digits; d >= 2; --d) {  // wave maxima, uniform
+    if (__any(dx >= d)) dx = max(dx, d);
+    if (__any(dw >= d)) dw = max(dw, d);
+  }
+  dx = __builtin_amdgcn_readfirstlane(dx);
+  dw = __builtin_amdgcn_readfirstlane(dw);
+  for (int s = 1; s <= min(dx + dw - 2, kI8Digits - 1); ++s)
+    for (int di = max(0, s - dw + 1); di <= min(s, dx - 1); ++di) product(di, s - di, std::false_type{});
 }
 
 // Rows and columns of a 32x32 block's accumulator: lane holds rows 8*(r/4) +
