@@ -67,7 +67,7 @@ constexpr int kMaxTail = 16;  // rows of the K tail (GemvF32Args::k_end - K)
 // read by the neighbouring block: plain loads, and neighbours on one XCD and
 // its L2 (16x4096x4097 21.4 us against 25.2 us streamed in launch order, and
 // 30.2 us for the aligned chunks realigned in registers that this replaced).
-template <int MB, int CPL, int WN, int WM>
+template <int MB, int CPL, int WN, int WM, int NS>
 __global__ void __launch_bounds__(waves_per_wg(MB, WN) * 64)
 gemv_f32_kernel(GemvF32Args a, int epi) {
   using vec = typename std::conditional<CPL == 4, f32x4u, f32x2u>::type;
@@ -109,11 +109,13 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
   const int li = lane & 15;
   const int lg = lane >> 4;
 
-  f32x4 acc[MB][CPL];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-    for (int c = 0; c < CPL; ++c) acc[mb][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  // NS = 2: steps alternate between two sets of accumulators, summed at the
+  // end: half the chain, 1/sqrt(2) of its rounding (relative 2-norm error
+  // against float64 at 16x4096x4096 2.1e-7 -> 1.5e-7, 16x8192x8192 4.1e-7 ->
+  // 2.9e-7). Three and four row blocks pay 3-4 % for it (64x8192x8192 93.5 ->
+  // 96.4 us) and take it where the plan splits K into fewer slices
+  // (GemvF32Args::two_sets).
+  f32x4 sum[NS][MB][CPL] = {};
 
   const int64_t ldw = a.ldw;
   const int col_lane = n0 + CPL * li;
@@ -162,7 +164,7 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
         x[u][mb] = f32x4{v[0], v[1], v[2], v[3]};
       }
   };
-  auto mfma_q = [&](const f32x4 (&xu)[MB], int s, const vec& wq) {
+  auto mfma_q = [&](f32x4 (&acc)[MB][CPL], const f32x4 (&xu)[MB], int s, const vec& wq) {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -188,7 +190,7 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
     int it = r0;
     load_x(x, it * 16 * kU);
     load_w(w, it * 16 * kU);
-    for (int i = 1; i < nit; ++i) {
+    auto iteration = [&](auto set) __attribute__((always_inline)) {
       int itn = it + 1;
       if (itn >= nit) itn = 0;
       const int kn = itn * 16 * kU;
@@ -196,7 +198,7 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
       const float* wp = wbase + (int64_t)kn * ldw;
 #pragma unroll
       for (int q = 0; q < 4 * kU; ++q) {
-        mfma_q(x[q / 4], q % 4, w[q]);
+        mfma_q(sum[(q / 4 + decltype(set)::value) % NS], x[q / 4], q % 4, w[q]);
         w[q] = load_row(wp + (int64_t)(16 * (q / 4) + q % 4) * ldw);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -205,9 +207,15 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) x[u][mb] = xn[u][mb];
       it = itn;
+    };
+    int i = 1;
+    for (; i + 1 < nit; i += 2) {
+      iteration(std::integral_constant<int, 0>{});
+      iteration(std::integral_constant<int, kU % 2>{});
     }
+    if (i < nit) iteration(std::integral_constant<int, 0>{});
 #pragma unroll
-    for (int q = 0; q < 4 * kU; ++q) mfma_q(x[q / 4], q % 4, w[q]);
+    for (int q = 0; q < 4 * kU; ++q) mfma_q(sum[(1 - q / 4) % NS], x[q / 4], q % 4, w[q]);
   }
   // Remaining single steps (kwave not a multiple of 16*kU).
   for (int k = nit * 16 * kU; k < kwave; k += 16) {
@@ -216,8 +224,15 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
     load_x(x, k);
     load_w(w, k);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) mfma_q(x[0], q, w[q]);
+    for (int q = 0; q < 4; ++q) mfma_q(sum[NS - 1], x[0], q, w[q]);
   }
+
+  f32x4 (&acc)[MB][CPL] = sum[0];
+  if constexpr (NS > 1)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) acc[mb][c] += sum[1][mb][c];
 
   // Sum the WK K-slices of each column block in wave order, one row block at
   // a time to bound LDS.
@@ -370,18 +385,25 @@ __global__ void __launch_bounds__(64) gemv_reduce_kernel(GemvF32Args a, int epi,
   }
 }
 
-template <int MB, int WM>
-hipError_t launch_mb_w(int cols, int epi, const GemvF32Args& a, hipStream_t stream) {
+template <int MB, int WM, int NS>
+hipError_t launch_mb_sets(int cols, int epi, const GemvF32Args& a, hipStream_t stream) {
   const dim3 grid(((a.N + cols - 1) / cols) * a.ksplit);
   auto block = [](int wn) { return dim3(waves_per_wg(MB, wn) * 64); };
   switch (cols) {
-    case 32: hipLaunchKernelGGL((gemv_f32_kernel<MB, 2, 1, WM>), grid, block(1), 0, stream, a, epi); break;
-    case 64: hipLaunchKernelGGL((gemv_f32_kernel<MB, 4, 1, WM>), grid, block(1), 0, stream, a, epi); break;
-    case 128: hipLaunchKernelGGL((gemv_f32_kernel<MB, 4, 2, WM>), grid, block(2), 0, stream, a, epi); break;
-    case 256: hipLaunchKernelGGL((gemv_f32_kernel<MB, 4, 4, WM>), grid, block(4), 0, stream, a, epi); break;
+    case 32: hipLaunchKernelGGL((gemv_f32_kernel<MB, 2, 1, WM, NS>), grid, block(1), 0, stream, a, epi); break;
+    case 64: hipLaunchKernelGGL((gemv_f32_kernel<MB, 4, 1, WM, NS>), grid, block(1), 0, stream, a, epi); break;
+    case 128: hipLaunchKernelGGL((gemv_f32_kernel<MB, 4, 2, WM, NS>), grid, block(2), 0, stream, a, epi); break;
+    case 256: hipLaunchKernelGGL((gemv_f32_kernel<MB, 4, 4, WM, NS>), grid, block(4), 0, stream, a, epi); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
+}
+
+template <int MB, int WM>
+hipError_t launch_mb_w(int cols, int epi, const GemvF32Args& a, hipStream_t stream) {
+  if constexpr (MB > 2 && WM != kWScalar)
+    if (!a.two_sets) return launch_mb_sets<MB, WM, 1>(cols, epi, a, stream);
+  return launch_mb_sets<MB, WM, 2>(cols, epi, a, stream);
 }
 
 template <int MB>

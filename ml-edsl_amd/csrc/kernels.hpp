@@ -74,6 +74,7 @@ struct GemvF32Args {
   const float* x_tail;
   int64_t ldx_tail;
   int k_end;
+  bool two_sets;      // two sets of accumulators for three and four row blocks too
   int w_mode;         // kWVector, kWShared or kWScalar (gemv_f32_w_mode)
 };
 
