@@ -9,6 +9,7 @@ seconds).
 from __future__ import annotations
 
 import concurrent.futures
+import importlib.util
 import os
 import shutil
 import subprocess
@@ -60,10 +61,12 @@ def build(jobs: int = 4, verbose: bool = False) -> str:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
-    ext = build_launch_module()
+    exts = [build_launch_module()]
+    if importlib.util.find_spec("torch") is not None:  # the device API needs torch, the host API does not
+        exts.append(build_torch_launch_module())
     if verbose:
-        print(f"built {LIB_PATH}")
-        print(f"built {ext}")
+        for path in [LIB_PATH, *exts]:
+            print(f"built {path}")
     return LIB_PATH
 
 
@@ -71,16 +74,32 @@ def build_launch_module() -> str:
     """The CPython binding of the device launch entries (csrc/pylaunch.c),
     linked against libedsl_hip.so next to it (found through $ORIGIN, so the
     process maps the one library that _native also loads)."""
-    import sysconfig
-    out = os.path.join(PKG_DIR, "_launch" + sysconfig.get_config_var("EXT_SUFFIX"))
-    tmp = out + ".tmp"
     cc = os.environ.get("CC") or shutil.which("gcc") or "cc"
-    cmd = [cc, "-O2", "-fPIC", "-shared", "-Wall", f"-I{sysconfig.get_paths()['include']}",
-           os.path.join(CSRC, "pylaunch.c"), "-o", tmp, f"-L{PKG_DIR}", "-l:" + LIB_NAME,
-           "-Wl,-rpath,$ORIGIN"]
+    return _link_module("_launch", [cc, "-O2", os.path.join(CSRC, "pylaunch.c")])
+
+
+def build_torch_launch_module() -> str:
+    """Its counterpart on torch tensors (csrc/torch_launch.cpp), linked against
+    torch's libraries, which the process has loaded before it imports this."""
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    cxx = os.environ.get("CXX") or shutil.which("g++") or "c++"
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    return _link_module("_torch_launch", [
+        cxx, "-O2", "-std=c++17", f"-D_GLIBCXX_USE_CXX11_ABI={abi}", *[f"-isystem{p}" for p in include_paths()],
+        os.path.join(CSRC, "torch_launch.cpp"), f"-L{libs}", "-ltorch_python", "-ltorch_cpu", "-lc10"])
+
+
+def _link_module(name: str, cmd: list[str]) -> str:
+    import sysconfig
+    out = os.path.join(PKG_DIR, name + sysconfig.get_config_var("EXT_SUFFIX"))
+    tmp = out + ".tmp"
+    cmd = [*cmd, "-fPIC", "-shared", "-Wall", f"-I{sysconfig.get_paths()['include']}", "-o", tmp, f"-L{PKG_DIR}",
+           "-l:" + LIB_NAME, "-Wl,-rpath,$ORIGIN"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
-        raise RuntimeError(f"building the launch module failed:\n{res.stdout}\n{res.stderr}")
+        raise RuntimeError(f"building {name} failed:\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, out)
     return out
 

@@ -10,6 +10,7 @@ from __future__ import annotations
 
 from . import _native
 
+_native_launch = None  # checks and launch on torch tensors (csrc/torch_launch.cpp), once loaded
 _launch = None  # METH_FASTCALL binding of the two entries (csrc/pylaunch.c), once loaded
 _torch = None
 _raw_stream = None  # (current device index) -> raw hipStream_t of that device's current stream
@@ -20,7 +21,7 @@ def _torch_module():
     current stream's raw handle: torch.cuda.current_stream() builds a Python
     stream object (~2.6 us per call on the GPU host), the raw accessor returns
     the same integer in ~0.1 us."""
-    global _torch, _raw_stream, _launch
+    global _torch, _raw_stream, _launch, _native_launch
     if _torch is None:
         import torch
         # The binding links the library: load it through _native first, which
@@ -31,6 +32,11 @@ def _torch_module():
             _launch = fast
         except ImportError:
             _launch = None
+        try:
+            from ._torch_launch import dense_launch as native_launch
+            _native_launch = native_launch
+        except ImportError:
+            _native_launch = None
         get_dev = getattr(torch._C, "_cuda_getDevice", None)
         get_raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
         if get_dev is not None and get_raw is not None:
@@ -73,6 +79,14 @@ def _validate(X, W, b, Y, torch) -> None:
 def dense_launch(X, W, b, Y, epilogue: int, alpha: float = 0.0, stream=None) -> None:
     """Y = epilogue(X @ W (+ b)); returns once the kernels are enqueued."""
     torch = _torch if _torch is not None else _torch_module()
+    if _native_launch is not None:
+        rc = _native_launch(X, W, b, Y, epilogue, alpha, stream, _raw_stream)
+        if rc == 0:
+            return
+        if rc is not None:
+            _native.raise_on_error("dense_launch")
+            return
+        # Not taken: tensor subclasses, or arguments that a check below refuses.
     dtype = X.dtype
     xs, ws = X.shape, W.shape
     # Everything _validate checks, as one short-circuit test of cheap tensor
