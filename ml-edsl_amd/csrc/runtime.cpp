@@ -298,6 +298,14 @@ void check_dims(int64_t M, int64_t N, int64_t K) {
          (long long)K);
 }
 
+// Bytes of the partial tiles of a small-M plan with `ks` splits. The automatic
+// plans keep them within the scratch of the allocation-free launch, which takes
+// the same plans.
+constexpr size_t kGemvFixedScratch = EDSL_NOALLOC_SCRATCH_BYTES;
+size_t gemv_partials(int ks, int64_t M, int64_t N) {
+  return (size_t)ks * 16 * ((M + 15) / 16) * ((N + 3) & ~int64_t(3)) * sizeof(float);
+}
+
 // Small-M plan. Widths are tried in the order 128, 256, 64, 32 columns per
 // workgroup. For each, the K split is the one of least cost: the time of the
 // rounds of workgroups over the CUs, in units of a full chip, plus the bytes
@@ -336,6 +344,7 @@ bool plan_gemv(const DeviceState& ds, int64_t M, int64_t N, int64_t K, int* cols
       if (chunks < 2 * wk) return false;
       double best = 0;
       for (int s = 1; s <= gemv_f32_max_ksplit() && chunks >= 2 * wk * s; ++s) {
+        if (s > 1 && gemv_partials(s, M, N) > kGemvFixedScratch) break;
         const int64_t rounds = (groups * s + ds.cus - 1) / ds.cus;
         const double cost = (double)(rounds * ds.cus) / (double)(groups * s) +
                             (s > 1 ? 2.0 * (double)s * (double)M / (double)K : 0.0);
@@ -396,7 +405,12 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
   const bool x_vec = al16(L.x) && L.ldx % 4 == 0;
   bool small_m = true;
   if (!w_vec)
-    small_m = K >= (row_blocks == 1 ? 384 : row_blocks == 2 ? 512 : 1024);
+    // (Where a K tail's two partials exceed the fixed scratch, from N = 32768 at
+    // M = 64: as long as the tiles, which need none, can have the layer.)
+    small_m = K >= (K % 16 && gemv_partials(2, M, N) > kGemvFixedScratch ? (row_blocks == 1 ? 1024 : 2048)
+                    : row_blocks == 1                                    ? 384
+                    : row_blocks == 2                                    ? 512
+                                                                         : 1024);
   else if (x_vec && row_blocks <= 3)
     small_m = K >= 512 << (row_blocks - 1);
   else if (x_vec)
@@ -451,9 +465,9 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
     a.alpha = L.alpha;
     a.ksplit = gemv_ks;
     a.ldp = ((int64_t)N + 3) & ~int64_t(3);
-    const int mb = (M + 15) / 16;
+    const int mb = row_blocks;
     const bool scratch = a.ksplit > 1;
-    const size_t part_bytes = scratch ? (size_t)a.ksplit * 16 * mb * a.ldp * sizeof(float) : 0;
+    const size_t part_bytes = scratch ? gemv_partials(a.ksplit, M, N) : 0;
     if (!has_bias) a.bias = nullptr;
     a.w_mode = gemv_f32_w_mode(a.W, a.ldw, N);
     // A split below the power of two that gives every CU a workgroup leaves

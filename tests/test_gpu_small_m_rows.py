@@ -42,3 +42,25 @@ def test_rows_of_any_alignment(M, K, N, pad, off):
     if pad:
         gap = ybuf[off:off + M * (N + pad)].view(M, N + pad)[:, N:]
         assert (gap == 7.0).all()
+
+
+# Wide N, where a split that fills the rounds of the CUs would need more than
+# the 16 MiB of partials that the allocation-free launch has: the automatic
+# plan, the same for both entries, stays within them.
+@pytest.mark.parametrize("M, K, N", [(48, 2048, 33024), (64, 1030, 40001), (16, 1024, 50257), (64, 2048, 8320)])
+def test_automatic_splits_fit_the_fixed_scratch(M, K, N):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(N)
+    X = torch.randn(M, K, device="cuda", generator=g)
+    W = torch.randn(K, N, device="cuda", generator=g)
+    b = torch.randn(N, device="cuda", generator=g)
+    Y, Z = torch.zeros(M, N, device="cuda"), torch.zeros(M, N, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    L = _native.lib()
+    for fn, out in ((L.edsl_hip_dense_f32_launch, Y), (L.edsl_hip_dense_f32_launch_noalloc, Z)):
+        rc = fn(X.data_ptr(), K, W.data_ptr(), N, b.data_ptr(), out.data_ptr(), N, M, N, K, _native.EPI_BIAS, 0.0,
+                stream)
+        assert rc == 0, _native.last_error()
+    torch.cuda.synchronize()
+    assert torch.equal(Y, Z)
+    assert torch.allclose(Y, torch.addmm(b, X, W), rtol=0, atol=1e-4 * K ** 0.5)
