@@ -473,8 +473,9 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
     // A split below the power of two that gives every CU a workgroup leaves
     // longer chains, which a second set of accumulators shortens again
     // (unaligned rows from 3/4 of it down: 48x4096x4097 on 7 of 8, 1.6e-7
-    // against float64 either way, is 4 % faster with one).
-    int full = 1;
+    // against float64 either way, is 4 % faster with one; one split has chains
+    // of all of K: 48x4096x50257 4.1e-7 with one set).
+    int full = w_vec ? 1 : 2;
     while (full < gemv_f32_max_ksplit() && ((int64_t)N + gemv_cols - 1) / gemv_cols * full < ds.cus) full *= 2;
     a.two_sets = w_vec ? a.ksplit < full : 4 * a.ksplit < 3 * full;
     if (fixed) {
