@@ -2,7 +2,8 @@
 """Benchmark of the dense hot path on one MI355X.
 
 Headline (BASELINE.json metric): fused fp32 matmul+bias+ReLU at M=N=K=4096
-(workload c3), in TFLOP/s and as a fraction of the dense fp32 MFMA peak.
+(workload c3), in TFLOP/s and as a fraction of the dense peak of the units its
+kernel runs on (six bf16 products per fp32 one).
 Secondary lines (same run): the M=16, K=N=8192 layer in GB/s (c4, W rotated
 over 3 buffers so the 256 MB Infinity Cache cannot serve it), the integer
 layer 2048^3 (c5, X and W rotated over 10 buffer pairs; the cache-resident

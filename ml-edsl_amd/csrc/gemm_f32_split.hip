@@ -41,14 +41,14 @@
 // only masked one. Rows past M and columns past N read the last row or column;
 // their outputs are not stored.
 //
-// What bounds it is power: the full chip runs this loop at 1.7-1.8 GHz, a
-// register-only loop of the same MFMAs takes 491 us of the 612 us at 4096^3,
-// and without the LDS reads the loop would take 470 (256x128 tiles of eight
-// waves). Hence the 256x256 tile of four waves, each 128x128: half the LDS
+// What bounds it is power: the full chip runs this loop at 1.8-1.87 GHz, a
+// register-only loop of the same MFMAs takes 491 us of the 574-583 us at
+// 4096^3, and without the LDS reads a loop on 256x128 tiles of eight waves took
+// 470 of 675-710. Hence the 256x256 tile of four waves, each 128x128: half the LDS
 // reads per MFMA of 64x64 wave tiles. Measured, us, against the fp32 tiles:
-// 4096^3 612 / 900 (225 TFLOP/s), 4000x1024x4000 177 / 224; 2048^3 on eight
-// waves of 64x32 97 / 117 (four waves of 64x64: 102), 2001^3 101 / 153;
-// 10000x500x1000 on two workgroups of 128x128x16 per CU 82 / 93.
+// 4096^3 574-583 / 907 (236-239 TFLOP/s), 4000x1024x4000 177 / 224; 2048^3 on
+// eight waves of 64x32 97 / 117 (four waves of 64x64: 102), 2001^3 97 / 154;
+// 10000x500x1000 on two workgroups of 128x128x16 per CU 78 / 94.
 #include "common.hpp"
 #include "kernels.hpp"
 

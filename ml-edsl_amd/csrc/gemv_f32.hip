@@ -19,7 +19,7 @@
 //    WK = NW/WN waves splitting the workgroup's K range. The WK slices are
 //    summed in LDS, in wave order. Fewer waves per CU keep fewer HBM rows
 //    open at once: 16-wave workgroups were 2-3 % slower at M=16, K=N=8192,
-//    6-10 % at M=48-64 and 10 % on realigned rows (16x8192x8191).
+//    6-10 % at M=48-64.
 //  * Wider column blocks read longer row runs but give fewer workgroups;
 //    they split K over `ksplit` workgroups to fill the chip. Each writes its
 //    partial tile, and a second small kernel sums the partials in split order
@@ -179,9 +179,8 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
   // iteration. (The scheduling barrier keeps the compiler from sinking the
   // reloads to the end of the iteration.) For three or four row blocks this
   // also measured faster than loading, waiting and computing one iteration at
-  // a time: at K = N = 8192, M = 48 80.5 vs 91.6 us and M = 64 104 vs 115 us
-  // (M = 64 with 4 columns per lane uses all 128 registers and 8-16 bytes of
-  // scratch); at K = N = 4096 the two measure the same.
+  // a time: at K = N = 8192, M = 48 80.5 vs 91.6 us and M = 64 104 vs 115 us;
+  // at K = N = 4096 the two measure the same.
   const int nit = kwave / (16 * kU);
   const int r0 = nit > 0 ? (int)(((unsigned)blockIdx.x * 2654435761u >> 8) + (unsigned)wk * 977u) % nit : 0;
   if (nit > 0) {
