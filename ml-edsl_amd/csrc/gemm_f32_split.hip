@@ -42,11 +42,11 @@
 // their outputs are not stored.
 //
 // What bounds it is power: the full chip runs this loop at 1.8-1.87 GHz, a
-// register-only loop of the same MFMAs takes 491 us of the 574-583 us at
+// register-only loop of the same MFMAs takes 491 us of the 574-587 us at
 // 4096^3, and without the LDS reads a loop on 256x128 tiles of eight waves took
 // 470 of 675-710. Hence the 256x256 tile of four waves, each 128x128: half the LDS
 // reads per MFMA of 64x64 wave tiles. Measured, us, against the fp32 tiles:
-// 4096^3 574-583 / 907 (236-239 TFLOP/s), 4000x1024x4000 177 / 224; 2048^3 on
+// 4096^3 574-587 / 907 (234-239 TFLOP/s), 4000x1024x4000 177 / 224; 2048^3 on
 // eight waves of 64x32 97 / 117 (four waves of 64x64: 102), 2001^3 97 / 154;
 // 10000x500x1000 on two workgroups of 128x128x16 per CU 78 / 94.
 #include "common.hpp"
