@@ -9,12 +9,25 @@
 // Every fp32 value is split exactly into three bf16 values, x = h + m + l (h
 // the nearest bf16 of x, m that of x - h, l the rest: 8 + 8 + 8 significand
 // bits), and the product takes six of the nine bf16 products, each exact in
-// fp32: hh, hm, mh, mm, hl, lh. The three left out are below 2^-25 of a
-// product. They are summed in fp32 by v_mfma_f32_32x32x16_bf16, smallest
-// first. Relative 2-norm error against float64, N(0,1) data, K = 1024 / 2048 /
-// 4096: with one accumulator (TWO false) 4.6e-7 / 6.3e-7 / 1.05e-6, with the
-// five small products in one of their own (TWO true) 1.7e-7 / 2.7e-7 /
-// 3.8e-7; the fp32 MFMA chain 5.8e-7 / 8.0e-7 / 1.14e-6.
+// fp32: hh, hm, mh, mm, hl, lh. They are summed in fp32 by
+// v_mfma_f32_32x32x16_bf16, hh in one accumulator and the small ones, smallest
+// first, in another, so that a step rounds the large sum once. (With all six in
+// one accumulator, six times: twice the fp32 chain's error on operands with a
+// nonzero value or two per step, 9.4e-7 against 8.1e-7 on X >= 0.)
+//
+// The products left out, ml, lm and ll, are below 2^-24 of a product together.
+// An fp32 chain of n terms is within n 2^-24 sum |ab| of the exact sum and this
+// one within 2 2^-24 of it, so only an output of a single term can lose by the
+// omission. Such an output has a row of A or a column of B with at most one
+// nonzero value. A workgroup therefore counts the nonzero values of its rows and
+// columns in the first three steps and, where one has fewer than two, takes
+// eight products (all but ll, below 2^-33).
+//
+// Relative 2-norm error against float64, this kernel / the fp32 MFMA chain:
+// N(0,1) data at K = 1024, 2048, 4096 1.9e-7 / 5.7e-7, 2.7e-7 / 8.1e-7, 4.0e-7
+// / 1.1e-6, after ReLU at K = 4096 3.2e-7 / 8.1e-7; rows with n nonzero values,
+// one per step, n = 1 2.5e-8 / 2.5e-8 (largest relative error 5.99e-8 / 5.96e-8),
+// n = 2 2.6e-8 / 3.1e-8, n = 8 2.9e-8 / 5.4e-8, n = 32 4.4e-8 / 1.03e-7.
 //
 // Not every value splits exactly (the last remainder of a value below 2^-109
 // leaves bf16's range; h overflows within half a bf16 step of the largest
@@ -42,13 +55,14 @@
 // their outputs are not stored.
 //
 // What bounds it is power: the full chip runs this loop at 1.8-1.87 GHz, a
-// register-only loop of the same MFMAs takes 491 us of the 574-587 us at
-// 4096^3, and without the LDS reads a loop on 256x128 tiles of eight waves took
-// 470 of 675-710. Hence the 256x256 tile of four waves, each 128x128: half the LDS
-// reads per MFMA of 64x64 wave tiles. Measured, us, against the fp32 tiles:
-// 4096^3 574-587 / 907 (234-239 TFLOP/s), 4000x1024x4000 177 / 224; 2048^3 on
-// eight waves of 64x32 97 / 117 (four waves of 64x64: 102), 2001^3 97 / 154;
-// 10000x500x1000 on two workgroups of 128x128x16 per CU 78 / 94.
+// register-only loop of the same MFMAs takes 491 us at 4096^3. The 256x128 tile
+// of four waves, each 128x64, reads LDS least of the tiles whose two sets of
+// accumulators fit the registers (a 256x256 tile with one took 580 us at the
+// error above). Measured, us, against the fp32 tiles: 4096^3 630-655 / 905
+// (210-218 TFLOP/s; 690 / 905 on eight products), 4000x1024x4000 176 / 240,
+// 2500^3 180 / 277; 2048^3 on eight waves of 64x32 96 / 120, 2001^3 99 / 159;
+// 10000x500x1000 on two workgroups of 128x128x16 per CU 78 / 94 (82 on eight
+// waves), 3333^3 428 / 681. Counting the first steps costs 1 % or less.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -88,12 +102,12 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&p)[kPlanes],
   }
 }
 
-// BM x BN outputs per workgroup of WM x WN waves, BK-deep steps of K. TWO: the
-// small products in their own accumulator.
-template <int BM_, int BN_, int WM_, int WN_, int BK_, bool TWO_>
+// BM x BN outputs per workgroup of WM x WN waves, BK-deep steps of K; WAVES on a
+// SIMD.
+template <int BM_, int BN_, int WM_, int WN_, int BK_, int WAVES_>
 struct SplitTile {
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, BK = BK_;
-  static constexpr bool TWO = TWO_;
+  static constexpr int kSimdWaves = WAVES_;
   static constexpr int kWaves = WM * WN;
   static constexpr int kThreads = 64 * kWaves;
   static constexpr int RB = BM / WM / 32, CB = BN / WN / 32;  // 32x32 blocks of a wave
@@ -168,10 +182,12 @@ __device__ __forceinline__ void fp32_wave_tile(const GemmF32Args& args, int m0, 
 }
 
 template <class C, int EPI>
-__global__ void __launch_bounds__(C::kThreads)
+__global__ void __launch_bounds__(C::kThreads, C::kSimdWaves)
 gemm_f32_split_kernel(GemmF32Args args) {
   constexpr int RB = C::RB, CB = C::CB, KK = C::KK;
   __shared__ __align__(16) char smem[C::kLds];
+  __shared__ int counts[C::BM + C::BN];  // nonzero values of the tile's rows and columns in the first steps
+  for (int i = threadIdx.x; i < C::BM + C::BN; i += C::kThreads) counts[i] = 0;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / C::WN, wn = wave % C::WN;
@@ -204,7 +220,7 @@ gemm_f32_split_kernel(GemmF32Args args) {
 
   constexpr int kOct = C::AO + C::BO;
   float raw[kOct][8];
-  auto load_octet = [&](int o, int k0) __attribute__((always_inline)) {
+  auto load_octet = [&](float (&raw)[kOct][8], int o, int k0) __attribute__((always_inline)) {
     if (o < C::AO) {
       const float* p = pa[o] + k0;
       const f32x4u v0 = *reinterpret_cast<const f32x4u*>(p), v1 = *reinterpret_cast<const f32x4u*>(p + 4);
@@ -238,27 +254,49 @@ gemm_f32_split_kernel(GemmF32Args args) {
     for (int q = 0; q < kPlanes; ++q) *reinterpret_cast<u32x4*>(st + at + q * C::kFrag) = p[q];
   };
 
-  f32x16 acc[RB][CB] = {};
-  f32x16 low[C::TWO ? RB : 1][C::TWO ? CB : 1] = {};
   // Steps: the K % BK rows first, if any, then the full steps.
   const int full = K / C::BK;
   const int has_tail = K % C::BK != 0;
   const int nit = full + has_tail;
   auto k_of = [&](int it) { return (min(it, nit - 1) - has_tail) * C::BK; };  // full steps
+  // The first kCheck full steps are loaded here for the count of their nonzero
+  // values, behind the first step, which is staged meanwhile.
+  constexpr int kCheck = C::BK == 16 ? 3 : 2;
+  float first[kCheck][kOct][8];
   if (has_tail) {
 #pragma unroll
     for (int o = 0; o < kOct; ++o) load_tail(o, full * C::BK);
   } else {
 #pragma unroll
-    for (int o = 0; o < kOct; ++o) load_octet(o, 0);
+    for (int o = 0; o < kOct; ++o) load_octet(raw, o, 0);
   }
+#pragma unroll
+  for (int c = 0; c < kCheck; ++c)
+#pragma unroll
+    for (int o = 0; o < kOct; ++o) load_octet(first[c], o, min(c, full - 1) * C::BK);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int o = 0; o < kOct; ++o) stage_octet(smem, o);
   if (nit > 1) {
 #pragma unroll
-    for (int o = 0; o < kOct; ++o) load_octet(o, k_of(1));
+    for (int o = 0; o < kOct; ++o) load_octet(raw, o, k_of(1));
+  }
+  __syncthreads();  // counts are zero
+#pragma unroll
+  for (int o = 0; o < kOct; ++o) {
+    int n = 0;
+#pragma unroll
+    for (int c = 0; c < kCheck; ++c)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) n += first[c][o][e] != 0.0f;
+    const int idx = o < C::AO ? ((int)threadIdx.x + o * C::kThreads) / C::OPR
+                              : C::BM + (wave + (o - C::AO) * C::kWaves) % (C::BN / 64) * 64 + lane;
+    atomicAdd(&counts[idx], n);
   }
   __syncthreads();
+  bool sparse = full < kCheck;  // its last step has been counted more than once
+  for (int i = threadIdx.x; i < C::BM + C::BN; i += C::kThreads) sparse |= counts[i] < 2;
+  const bool eight = __syncthreads_or(sparse) != 0;  // uniform: take ml and lm
 
   constexpr int BS = KK == 1 ? 2 : KK;  // sets of B fragments
   bf16x8 a[2][kPlanes], b[BS][CB][kPlanes];
@@ -284,101 +322,106 @@ gemm_f32_split_kernel(GemmF32Args args) {
   static_assert(kSlices % 2 == 0, "A sets alternate by slice");
   read_a(smem, 0, 0);
   read_b(smem, 0, 0);
-  auto step = [&](int it, auto set_c) __attribute__((always_inline)) {
-    constexpr int S = decltype(set_c)::value;  // parity of the step
-    const char* st = smem + S * C::kStage;
-    char* sn = smem + (S ^ 1) * C::kStage;
-    const int k2 = k_of(it + 2);
+  // The K loop on PRODUCTS (6 or 8) products and the stores; false, with nothing
+  // stored, if the tile must be recomputed.
+  auto compute = [&](auto products_c) __attribute__((always_inline)) {
+    constexpr int PRODUCTS = decltype(products_c)::value;
+    f32x16 acc[RB][CB] = {}, low[RB][CB] = {};
+    auto step = [&](int it, auto set_c) __attribute__((always_inline)) {
+      constexpr int S = decltype(set_c)::value;  // parity of the step
+      const char* st = smem + S * C::kStage;
+      char* sn = smem + (S ^ 1) * C::kStage;
+      const int k2 = k_of(it + 2);
 #pragma unroll
-    for (int sl = 0; sl < kSlices; ++sl) {
-      const int i = sl / KK, kk = sl % KK;
-      const int bs = KK == 1 ? S : kk;
-      if (sl == kSlices - 1) {
-        __syncthreads();
-        read_a(sn, 0, (sl + 1) & 1);
-        read_b(sn, 0, KK == 1 ? S ^ 1 : 0);
-      } else {
-        read_a(st, sl + 1, (sl + 1) & 1);
-        if (i == 0 && kk + 1 < KK) read_b(st, kk + 1, kk + 1);
-      }
-      // Smallest products first.
-      constexpr int pa_[6] = {2, 0, 1, 1, 0, 0}, pb_[6] = {0, 2, 1, 0, 1, 0};
-#pragma unroll
-      for (int s = 0; s < 6; ++s)
-#pragma unroll
-        for (int j = 0; j < CB; ++j) {
-          f32x16& t = C::TWO && s < 5 ? low[C::TWO ? i : 0][C::TWO ? j : 0] : acc[i][j];
-          t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[sl & 1][pa_[s]], b[bs][j][pb_[s]], t, 0, 0, 0);
+      for (int sl = 0; sl < kSlices; ++sl) {
+        const int i = sl / KK, kk = sl % KK;
+        const int bs = KK == 1 ? S : kk;
+        if (sl == kSlices - 1) {
+          __syncthreads();
+          read_a(sn, 0, (sl + 1) & 1);
+          read_b(sn, 0, KK == 1 ? S ^ 1 : 0);
+        } else {
+          read_a(st, sl + 1, (sl + 1) & 1);
+          if (i == 0 && kk + 1 < KK) read_b(st, kk + 1, kk + 1);
         }
-      if (sl < kSlices - 1) {
-        // Octets sl, sl + (kSlices - 1), ... of the next stage; each one's
-        // registers are then free for the octet of the step after.
+        // Smallest products first.
+        constexpr int pa_[8] = {1, 2, 2, 0, 1, 1, 0, 0}, pb_[8] = {2, 1, 0, 2, 1, 0, 1, 0};
 #pragma unroll
-        for (int o = sl; o < kOct; o += kSlices - 1) {
-          stage_octet(sn, o);
-          load_octet(o, k2);
+        for (int s = 8 - PRODUCTS; s < 8; ++s)
+#pragma unroll
+          for (int j = 0; j < CB; ++j) {
+            f32x16& t = s < 7 ? low[i][j] : acc[i][j];
+            t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[sl & 1][pa_[s]], b[bs][j][pb_[s]], t, 0, 0, 0);
+          }
+        if (sl < kSlices - 1) {
+          // Octets sl, sl + (kSlices - 1), ... of the next stage; each one's
+          // registers are then free for the octet of the step after.
+#pragma unroll
+          for (int o = sl; o < kOct; o += kSlices - 1) {
+            stage_octet(sn, o);
+            load_octet(raw, o, k2);
+          }
         }
-      }
-      // One MFMA, at most one LDS read, five VALU operations, and so on: the
-      // compiler otherwise puts the splitting after the MFMAs.
-      constexpr int kReads[2] = {3, 3 + 3 * CB};
-      const int reads = kReads[sl == kSlices - 1 || (i == 0 && kk + 1 < KK)];
+        // One MFMA, at most one LDS read, five VALU operations, and so on: the
+        // compiler otherwise puts the splitting after the MFMAs.
+        constexpr int kReads[2] = {3, 3 + 3 * CB};
+        const int reads = kReads[sl == kSlices - 1 || (i == 0 && kk + 1 < KK)];
 #pragma unroll
-      for (int m = 0; m < 6 * CB; ++m) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (m < reads) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+        for (int m = 0; m < PRODUCTS * CB; ++m) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          if (m < reads) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);
+    };
+    int it = 0;
+    for (; it + 1 < nit; it += 2) {
+      step(it, std::integral_constant<int, 0>{});
+      step(it + 1, std::integral_constant<int, 1>{});
     }
-  };
-  int it = 0;
-  for (; it + 1 < nit; it += 2) {
-    step(it, std::integral_constant<int, 0>{});
-    step(it + 1, std::integral_constant<int, 1>{});
-  }
-  if (it < nit) step(it, std::integral_constant<int, 0>{});
+    if (it < nit) step(it, std::integral_constant<int, 0>{});
 
-  if constexpr (C::TWO)
 #pragma unroll
     for (int i = 0; i < RB; ++i)
 #pragma unroll
       for (int j = 0; j < CB; ++j) acc[i][j] += low[i][j];
-  bool bad = (lost & 0xffffu) != 0;
+    bool bad = (lost & 0xffffu) != 0;
 #pragma unroll
-  for (int i = 0; i < RB; ++i)
+    for (int i = 0; i < RB; ++i)
 #pragma unroll
-    for (int j = 0; j < CB; ++j)
+      for (int j = 0; j < CB; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) bad |= !(__builtin_fabsf(acc[i][j][e]) < __builtin_huge_valf());
-  if (__syncthreads_or(bad)) {  // uniform
-    fp32_wave_tile<C, EPI>(args, m0 + wm * RB * 32, n0 + wn * CB * 32);
-    return;
-  }
-  // Lane: rows 8 (r/4) + 4 (lane/32) + r%4 and column lane%32 of a block, so
-  // each store writes two 128-byte row segments. The stores go through a
-  // descriptor of C's rows m0 .. M-1, whose range check drops rows past M;
-  // columns past N are sent out of range. (A branch per store cost an edge
-  // tile 20 us; ldc is below 2^21, so a tile's offsets fit 31 bits.)
-  const int half = lane >> 5, l32 = lane & 31;
-  const int ldc = (int)args.ldc;
-  const i32x4 rsrc = buffer_rsrc(args.C + (int64_t)m0 * ldc, (int64_t)(M - m0) * ldc * 4);
+        for (int e = 0; e < 16; ++e) bad |= !(__builtin_fabsf(acc[i][j][e]) < __builtin_huge_valf());
+    if (__syncthreads_or(bad)) return false;  // uniform
+    // Lane: rows 8 (r/4) + 4 (lane/32) + r%4 and column lane%32 of a block, so
+    // each store writes two 128-byte row segments. The stores go through a
+    // descriptor of C's rows m0 .. M-1, whose range check drops rows past M;
+    // columns past N are sent out of range. (A branch per store cost an edge
+    // tile 20 us; ldc is below 2^21, so a tile's offsets fit 31 bits.)
+    const int half = lane >> 5, l32 = lane & 31;
+    const int ldc = (int)args.ldc;
+    const i32x4 rsrc = buffer_rsrc(args.C + (int64_t)m0 * ldc, (int64_t)(M - m0) * ldc * 4);
 #pragma unroll
-  for (int j = 0; j < CB; ++j) {
-    const int col = n0 + (wn * CB + j) * 32 + l32;
-    const float bv = epi_has_bias(EPI) && col < N ? args.bias[col] : 0.0f;
+    for (int j = 0; j < CB; ++j) {
+      const int col = n0 + (wn * CB + j) * 32 + l32;
+      const float bv = epi_has_bias(EPI) && col < N ? args.bias[col] : 0.0f;
 #pragma unroll
-    for (int i = 0; i < RB; ++i) {
-      const int at = (((wm * RB + i) * 32 + 4 * half) * ldc + col) * 4;
+      for (int i = 0; i < RB; ++i) {
+        const int at = (((wm * RB + i) * 32 + 4 * half) * ldc + col) * 4;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int dr = 8 * (r >> 2) + (r & 3);
-        raw_buffer_store_f32(apply_epilogue_f32<EPI>(acc[i][j][r], bv, args.alpha), rsrc,
-                             col < N ? at + dr * ldc * 4 : 0x7fffffff, 0, kAuxNonTemporal);
+        for (int r = 0; r < 16; ++r) {
+          const int dr = 8 * (r >> 2) + (r & 3);
+          raw_buffer_store_f32(apply_epilogue_f32<EPI>(acc[i][j][r], bv, args.alpha), rsrc,
+                               col < N ? at + dr * ldc * 4 : 0x7fffffff, 0, kAuxNonTemporal);
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);
     }
-  }
+    return true;
+  };
+  const bool done = eight ? compute(std::integral_constant<int, 8>{}) : compute(std::integral_constant<int, 6>{});
+  if (!done) fp32_wave_tile<C, EPI>(args, m0 + wm * RB * 32, n0 + wn * CB * 32);
 }
 
 template <class C>
@@ -408,9 +451,9 @@ hipError_t launch_tile(int epi, GemmF32Args a, hipStream_t stream) {
 hipError_t launch_gemm_f32_split(int tile, int epi, GemmF32Args a, hipStream_t stream) {
   if (a.M < 1 || a.N < 1 || a.K < 32 || a.ldc >= kF32SplitMaxLdc) return hipErrorInvalidValue;  // a full step of K
   switch (tile) {
-    case kSplit256: return launch_tile<SplitTile<256, 256, 2, 2, 16, false>>(epi, a, stream);
-    case kSplit128W8: return launch_tile<SplitTile<128, 128, 2, 4, 32, true>>(epi, a, stream);
-    case kSplit128Pair: return launch_tile<SplitTile<128, 128, 2, 2, 16, false>>(epi, a, stream);
+    case kSplit256x128: return launch_tile<SplitTile<256, 128, 2, 2, 16, 1>>(epi, a, stream);
+    case kSplit128W8: return launch_tile<SplitTile<128, 128, 2, 4, 32, 2>>(epi, a, stream);
+    case kSplit128Pair: return launch_tile<SplitTile<128, 128, 2, 2, 16, 2>>(epi, a, stream);
     default: return hipErrorInvalidValue;
   }
 }

@@ -401,7 +401,7 @@ int plan_f32_small(const F32TileQuery& q, bool stream_rows) {
 
 const char* f32_split_name(int tile) {
   switch (tile) {
-    case kSplit256: return "256x256x16";
+    case kSplit256x128: return "256x128x16";
     case kSplit128W8: return "128x128x32_w8";
     case kSplit128Pair: return "128x128x16";
     default: return "none";
@@ -409,8 +409,8 @@ const char* f32_split_name(int tile) {
 }
 
 int64_t f32_split_grid(int tile, int64_t M, int64_t N) {
-  const int64_t b = tile == kSplit256 ? 256 : 128;
-  return ((M + b - 1) / b) * ((N + b - 1) / b);
+  const int64_t bm = tile == kSplit256x128 ? 256 : 128;
+  return ((M + bm - 1) / bm) * ((N + 127) / 128);
 }
 
 int plan_f32_split(const F32TileQuery& q, int cfg) {
@@ -420,40 +420,40 @@ int plan_f32_split(const F32TileQuery& q, int cfg) {
   const int64_t tiles = ((q.M + g.bm - 1) / g.bm) * ((q.N + g.bn - 1) / g.bn);
   auto rounds = [](int64_t n, double slots) { return (double)(int64_t)(((double)n + slots - 1) / slots); };
   // The fp32 tile's time in us, from its time per round of workgroups and k
-  // (4096^3 902 us in one round of 128x128, 465 in each of two of 128x256,
-  // 2048^3 117 on unsplit 64x64, 1024^3 18 on K-split 64x64, 2001^3 153 and
-  // 4001^3 1116 on any-shape tiles, 2000^3 137 on 128x128 of eight waves).
-  // `chain`: K is summed in one chain, whose error one accumulator of the
-  // split product stays below; tiles that split K need the two of kSplit128W8.
-  bool chain = true;
+  // (4096^3 902 us and 4096x256x4096 69 in one round of 128x128, 465 and
+  // 5982x272x3844 42 in each round of 128x256, 2048^3 117 on unsplit 64x64,
+  // 2001^3 153 and 4001^3 1116 on any-shape tiles, 2000^3 137 on 128x128 of eight
+  // waves; 3072^3 393 us and 2944x256x3968 63 in 9 and 12 rounds of K-split 64x64,
+  // 3620x1708x640 84 and 1744x260x3832 45 in 3 and 7 of 64x64 edge tiles,
+  // 3516x1629x1353 165 and 4651x263x947 42 in 5 of any-shape 64x64).
   double f32_us;
   switch (cfg) {
-    case kF32Direct128: case kF32Direct128Edge: f32_us = rounds(tiles, 4 * cus) * 0.220 * K; break;
+    case kF32Direct128: case kF32Direct128Edge: f32_us = rounds(tiles, 4 * cus) * (0.216 * K + 14); break;
     case kF32Direct64: f32_us = rounds(tiles, 4 * cus) * 0.057 * K; break;
-    case kF32M16_128x256: case kF32M16_128x256Edge: f32_us = rounds(tiles, cus) * 0.1135 * K; break;
+    case kF32M16_128x256: case kF32M16_128x256Edge: f32_us = rounds(tiles, cus) * (0.1107 * K + 12); break;
     case kF32M16_128: case kF32M16_128Edge: case kF32M16_128W8: case kF32M16_128W8Edge: {
       const double n = rounds(tiles, cus);
       f32_us = ((double)((int64_t)n / 2) * 0.126 + (double)((int64_t)n % 2) * 0.067) * K;
       break;
     }
-    case kF32M16_64: case kF32M16_64Edge: f32_us = rounds(tiles, cus) * 0.0172 * K; break;
+    case kF32M16_64: case kF32M16_64Edge: f32_us = rounds(tiles, cus) * (0.0166 * K + 1.7); break;
     case kF32T256Any: f32_us = rounds(tiles, cus) * 0.275 * K; break;
     case kF32M16_128Any: f32_us = rounds(tiles, cus) * 0.0745 * K; break;
     case kF32Direct64K4: case kF32Direct64K4Edge: case kF32DirectRC4x4: case kF32DirectRC4x4Edge:
     case kF32DirectRC5x5: case kF32DirectRC5x5Edge: case kF32DirectRC6x6: case kF32DirectRC6x6Edge:
-      chain = false;
-      f32_us = rounds(tiles, cus) * 0.0146 * K * (double)(g.bm * g.bn) / 4096.0;
+      f32_us = rounds(tiles, cus) * (0.0139 * K + 1.6) * (double)(g.bm * g.bn) / 4096.0;
       break;
     case kF32T64Any: case kF32T64K2Any:
-      chain = false;
-      f32_us = rounds(tiles, cus) * 0.024 * K;
+      f32_us = rounds(tiles, cus) * (0.019 * K + 2.6);
       break;
     default: return kSplitNone;
   }
-  // The split tiles' times: 4096^3 612 us in one round of 256x256, 2048^3 97
-  // in one of 128x128 on eight waves; two 128x128x16 workgroups on a CU take
-  // 2.8 us per 32 k, one alone 1.7 (4096^3 722 us, 10000x500x1000 82).
-  const int64_t t256 = f32_split_grid(kSplit256, q.M, q.N), t128 = f32_split_grid(kSplit128W8, q.M, q.N);
+  // The split tiles' times: 4096^3 655 us in two rounds of 256x128, 2500^3 180 in
+  // one, 4000x1024x4000 176 in two; on 128x128 of eight waves 2048^3 96 us in one
+  // round, 10000x500x1000 81 and 5806x372x1727 63 in three; two 128x128x16
+  // workgroups on a CU 2048x4096x4096 340 us and 4096^3 696, one alone 2048^3 100,
+  // both 10000x500x1000 78 and 5806x372x1727 69.
+  const int64_t t256 = f32_split_grid(kSplit256x128, q.M, q.N), t128 = f32_split_grid(kSplit128W8, q.M, q.N);
   const double n128 = rounds(t128, cus);
   double best_us = 0.93 * f32_us;
   int best = kSplitNone;
@@ -463,12 +463,10 @@ int plan_f32_split(const F32TileQuery& q, int cfg) {
       best = tile;
     }
   };
-  consider(kSplit128W8, n128 * 0.0453 * K + 5);
-  if (chain) {
-    consider(kSplit256, rounds(t256, cus) * 0.148 * K + 10);
-    consider(kSplit128Pair,
-             ((double)((int64_t)n128 / 2) * 0.0875 + (double)((int64_t)n128 % 2) * 0.053) * K + 8);
-  }
+  consider(kSplit128W8, n128 * (0.0435 * K + 3.5) + 3);
+  consider(kSplit256x128, rounds(t256, cus) * (0.076 * K + 10));
+  consider(kSplit128Pair, (double)((int64_t)n128 / 2) * (0.080 * K + 6.5) +
+                              (double)((int64_t)n128 % 2) * (0.046 * K + 6) + 3);
   return best;
 }
 

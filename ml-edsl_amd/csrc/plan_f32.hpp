@@ -109,9 +109,9 @@ bool gemm_f32_direct_offsets_fit(int64_t K, int64_t lda, int64_t ldb);
 // The tiles on bf16 matrix cores at fp32 precision (gemm_f32_split.hip).
 enum F32SplitTile : int {
   kSplitNone = -1,
-  kSplit256 = 0,   // 256x256x16, four waves, one workgroup per CU, one accumulator
-  kSplit128W8,     // 128x128x32, eight waves, one workgroup per CU, two accumulators
-  kSplit128Pair,   // 128x128x16, four waves, two workgroups per CU, one accumulator
+  kSplit256x128 = 0,  // 256x128x16, four waves, one workgroup per CU
+  kSplit128W8,        // 128x128x32, eight waves, one workgroup per CU
+  kSplit128Pair,      // 128x128x16, four waves, two workgroups per CU
 };
 // The split tile for a layer whose fp32 tile is `cfg` (plan_f32_tile), or
 // kSplitNone where the fp32 tile is the better one.

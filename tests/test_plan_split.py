@@ -37,18 +37,18 @@ def driver(tmp_path_factory):
 
 # (M, K, N), aligned, forced configuration, ldc (0: N), split tile
 CASES = [
-    ((4096, 4096, 4096), 1, -1, 0, "256x256x16"), ((4096, 256, 4096), 1, -1, 0, "256x256x16"),
-    ((4001, 4001, 4001), 0, -1, 0, "256x256x16"), ((4000, 1024, 4000), 1, -1, 0, "256x256x16"),
+    ((4096, 4096, 4096), 1, -1, 0, "256x128x16"), ((4096, 256, 4096), 1, -1, 0, "128x128x16"),
+    ((4001, 4001, 4001), 0, -1, 0, "256x128x16"), ((4000, 1024, 4000), 1, -1, 0, "256x128x16"),
+    ((2500, 2500, 2500), 1, -1, 0, "256x128x16"), ((2048, 4096, 4096), 1, -1, 0, "256x128x16"),
     ((2048, 2048, 2048), 1, -1, 0, "128x128x32_w8"), ((2001, 2001, 2001), 0, -1, 0, "128x128x32_w8"),
-    ((10000, 500, 1000), 1, -1, 0, "128x128x32_w8"),
-    ((2048, 4096, 4096), 1, -1, 0, "128x128x16"), ((2500, 2500, 2500), 1, -1, 0, "128x128x16"),
-    # K split over waves: the fp32 tile's shorter chains and even rounds are kept
+    ((10000, 500, 1000), 1, -1, 0, "128x128x16"), ((3333, 3333, 3333), 0, -1, 0, "128x128x16"),
+    # K split over waves in even rounds
     ((1024, 1024, 1024), 1, -1, 0, "none"), ((3072, 3072, 3072), 1, -1, 0, "none"),
     ((1500, 1500, 1500), 1, -1, 0, "none"), ((1000, 1000, 1000), 1, -1, 0, "none"),
     # short K, small M, a forced configuration, rows of C past 31-bit offsets
     ((4096, 255, 4096), 1, -1, 0, "none"), ((64, 4096, 8192), 1, -1, 0, "none"),
     ((4096, 4096, 4096), 1, 16, 0, "none"), ((4096, 4096, 4096), 1, -1, 1 << 21, "none"),
-    ((4096, 4096, 4096), 1, -1, (1 << 21) - 1, "256x256x16"),
+    ((4096, 4096, 4096), 1, -1, (1 << 21) - 1, "256x128x16"),
 ]
 
 
