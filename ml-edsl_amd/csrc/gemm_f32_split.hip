@@ -29,14 +29,23 @@
 // one per step, n = 1 2.5e-8 / 2.5e-8 (largest relative error 5.99e-8 / 5.96e-8),
 // n = 2 2.6e-8 / 3.1e-8, n = 8 2.9e-8 / 5.4e-8, n = 32 4.4e-8 / 1.03e-7.
 //
-// Not every value splits exactly (the last remainder of a value below 2^-109
-// leaves bf16's range; h overflows within half a bf16 step of the largest
-// float), Inf - Inf is NaN, and a partial sum may overflow in one order and not
-// in another. A workgroup therefore ORs the low halves of all its last
-// remainders (zero exactly when they are bf16 values) and, at the end, tests
-// its sums; if any remainder was cut or any sum is not finite it recomputes its
-// tile on v_mfma_f32_16x16x4_f32 from the fp32 operands, with that path's
-// results for denormal, huge, infinite and NaN values.
+// Not every value splits exactly. Below 2^-109 the last remainder may leave
+// bf16's range, which cuts at most 2^-134 off the value; near the largest float
+// h overflows; and where sums are below 2^-126, rounding is no longer relative
+// (2^-150 each; the matrix cores keep subnormal operands and results). A
+// workgroup ORs the low halves of all its last remainders (zero exactly when
+// they are bf16 values), keeps its largest value, and at the end tests its sums.
+// One that is not finite, or is smaller than 2^26 times what may have been lost
+// -- K 2^-150 from underflow, and with a value cut K 2^-133 times the largest
+// value, unless its row or column is zero throughout -- sends the whole tile to
+// v_mfma_f32_16x16x4_f32 and the fp32 operands, with that path's results for
+// denormal, huge, infinite and NaN values. So denormals among ordinary values
+// are nearly free (one in every row: 4096^3 662 -> 682 us, 2048^3 97 -> 102; 783
+// and 105 with rows of zeros as well; sending every tile with a cut value to a
+// loop without LDS took 2411 and 542), and a layer whose every tile holds an
+// infinity, a NaN or a value near the largest float, or whose sums are all tiny,
+// pays for both: 4096^3 1760 us, 2048^3 240, 10000x500x1000 190, twice the fp32
+// tiles' time.
 //
 // Bounds and layout. Splitting costs six VALU operations an element, so it is
 // done once per workgroup, on the way into LDS, never per wave: eight k of a
@@ -58,11 +67,12 @@
 // register-only loop of the same MFMAs takes 491 us at 4096^3. The 256x128 tile
 // of four waves, each 128x64, reads LDS least of the tiles whose two sets of
 // accumulators fit the registers (a 256x256 tile with one took 580 us at the
-// error above). Measured, us, against the fp32 tiles: 4096^3 630-655 / 905
-// (210-218 TFLOP/s; 690 / 905 on eight products), 4000x1024x4000 176 / 240,
-// 2500^3 180 / 277; 2048^3 on eight waves of 64x32 96 / 120, 2001^3 99 / 159;
-// 10000x500x1000 on two workgroups of 128x128x16 per CU 78 / 94 (82 on eight
-// waves), 3333^3 428 / 681. Counting the first steps costs 1 % or less.
+// error above). Measured, us, against the fp32 tiles: 4096^3 650-662 / 905
+// (208-211 TFLOP/s; 700 / 905 on eight products), 4000x1024x4000 178 / 245,
+// 2500^3 184 / 277; 2048^3 on eight waves of 64x32 97 / 120, 2001^3 99 / 159;
+// 10000x500x1000 on two workgroups of 128x128x16 per CU 75 / 94 (83 on eight
+// waves), 3333^3 428 / 681. Counting the first steps and testing the sums cost
+// 1 % or less.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -86,8 +96,9 @@ __device__ __forceinline__ uint32_t cvt_pk_bf16(float a, float b) {
 __device__ __forceinline__ float bf_lo(uint32_t p) { return __builtin_bit_cast(float, p << 16); }
 __device__ __forceinline__ float bf_hi(uint32_t p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
 
-// Eight floats as three bf16 planes; ORs the bits of the last remainders into `lost`.
-__device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&p)[kPlanes], uint32_t& lost) {
+// Eight floats as three bf16 planes; ORs the bits of the last remainders into
+// `lost` and keeps the largest magnitude of the first plane in `big`.
+__device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&p)[kPlanes], uint32_t& lost, float& big) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const float a = x[2 * i], b = x[2 * i + 1];
@@ -99,15 +110,17 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&p)[kPlanes],
     p[1][i] = m;
     p[2][i] = cvt_pk_bf16(qa, qb);
     lost |= __builtin_bit_cast(uint32_t, qa) | __builtin_bit_cast(uint32_t, qb);
+    const f32x2 hf = __builtin_convertvector(__builtin_bit_cast(bf16x2, h), f32x2);
+    big = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(hf[0]), __builtin_fabsf(hf[1])), big);
   }
 }
 
 // BM x BN outputs per workgroup of WM x WN waves, BK-deep steps of K; WAVES on a
-// SIMD.
-template <int BM_, int BN_, int WM_, int WN_, int BK_, int WAVES_>
+// SIMD, VALU operations scheduled behind an MFMA.
+template <int BM_, int BN_, int WM_, int WN_, int BK_, int WAVES_, int VALU_>
 struct SplitTile {
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, BK = BK_;
-  static constexpr int kSimdWaves = WAVES_;
+  static constexpr int kSimdWaves = WAVES_, kValu = VALU_;
   static constexpr int kWaves = WM * WN;
   static constexpr int kThreads = 64 * kWaves;
   static constexpr int RB = BM / WM / 32, CB = BN / WN / 32;  // 32x32 blocks of a wave
@@ -124,61 +137,77 @@ struct SplitTile {
   static_assert(BN % 64 == 0 && BM % 32 == 0, "tile");
 };
 
-// A wave's outputs from row m0 and column n0 on, from the fp32 operands on
-// v_mfma_f32_16x16x4_f32: a workgroup whose values do not all split exactly,
-// or whose sums are not all finite, recomputes its tile here.
-// 64 rows at a time (128 x 128 accumulators at once would spill).
-template <class C, int EPI>
-__device__ __forceinline__ void fp32_wave_rows(const GemmF32Args& args, int m0, int n0) {
-  constexpr int R = 4, CC = 2 * C::CB;  // 16x16 blocks
+// The tile from the fp32 operands on v_mfma_f32_16x16x4_f32, for a workgroup
+// whose values do not allow the split. `load` fetches a step's octets into
+// registers; they are staged in LDS as [k][row] and [k][column], whose pitches
+// put the four k of an MFMA operand on different banks.
+template <class C, int EPI, class Load>
+__device__ __forceinline__ void fp32_tile(const GemmF32Args& args, char* smem, int m0, int n0, int nit,
+                                          float (&raw)[C::AO + C::BO][8], Load load) {
+  constexpr int R = 2 * C::RB, CC = 2 * C::CB;  // 16x16 blocks of a wave
+  constexpr int PA = C::BM + 16, PB = C::BN + 16;
+  constexpr int kBuf = C::BK * (PA + PB);
+  static_assert(2 * kBuf * 4 <= C::kLds, "two stages of fp32 operands");
+  float* lds = reinterpret_cast<float*>(smem);
   const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / C::WN * C::RB * 32, wn = wave % C::WN * C::CB * 32;
   const int g = lane >> 4, r16 = lane & 15;
-  const int M = args.M, N = args.N, K = args.K;
-  const float* pa[R];
-  int col[CC];
+  auto stage = [&](float* st) __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < R; ++i) pa[i] = args.A + (int64_t)min(m0 + 16 * i + r16, M - 1) * args.lda;
+    for (int i = 0; i < C::AO; ++i) {
+      const int idx = threadIdx.x + i * C::kThreads;
+      float* p = st + 8 * (idx % C::OPR) * PA + idx / C::OPR;
 #pragma unroll
-  for (int c = 0; c < CC; ++c) col[c] = min(n0 + 16 * c + r16, N - 1);
+      for (int e = 0; e < 8; ++e) p[e * PA] = raw[i][e];
+    }
+#pragma unroll
+    for (int i = 0; i < C::BO; ++i) {
+      const int idx = wave + i * C::kWaves;
+      float* p = st + C::BK * PA + 8 * (idx / (C::BN / 64)) * PB + idx % (C::BN / 64) * 64 + lane;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) p[e * PB] = raw[C::AO + i][e];
+    }
+  };
   f32x4 acc[R][CC] = {};
+  load(0);
+  stage(lds);
+  load(1);
+  __syncthreads();
 #pragma unroll 1
-  for (int k0 = 0; k0 < K; k0 += 4) {
-    const int k = k0 + g, kc = min(k, K - 1);
-    const float* pb = args.B + (int64_t)kc * args.ldb;
-    float a[R], b[CC];
+  for (int it = 0; it < nit; ++it) {
+    const float* st = lds + (it & 1) * kBuf;
+    const float* sa = st + g * PA + wm + r16;
+    const float* sb = st + C::BK * PA + g * PB + wn + r16;
 #pragma unroll
-    for (int i = 0; i < R; ++i) a[i] = pa[i][kc];
+    for (int k = 0; k < C::BK; k += 4) {
+      float a[R], b[CC];
 #pragma unroll
-    for (int c = 0; c < CC; ++c) b[c] = pb[col[c]];
+      for (int i = 0; i < R; ++i) a[i] = sa[k * PA + 16 * i];
 #pragma unroll
-    for (int i = 0; i < R; ++i) a[i] = k < K ? a[i] : 0.0f;
+      for (int c = 0; c < CC; ++c) b[c] = sb[k * PB + 16 * c];
 #pragma unroll
-    for (int c = 0; c < CC; ++c) b[c] = k < K ? b[c] : 0.0f;
+      for (int i = 0; i < R; ++i)
 #pragma unroll
-    for (int i = 0; i < R; ++i)
-#pragma unroll
-      for (int c = 0; c < CC; ++c) acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[c], acc[i][c], 0, 0, 0);
+        for (int c = 0; c < CC; ++c) acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[c], acc[i][c], 0, 0, 0);
+    }
+    stage(lds + ((it + 1) & 1) * kBuf);
+    load(it + 2);
+    __syncthreads();
   }
 #pragma unroll
   for (int c = 0; c < CC; ++c) {
-    const int n = n0 + 16 * c + r16;
-    if (n >= N) continue;
+    const int n = n0 + wn + 16 * c + r16;
+    if (n >= args.N) continue;
     const float bv = epi_has_bias(EPI) ? args.bias[n] : 0.0f;
 #pragma unroll
     for (int i = 0; i < R; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int m = m0 + 16 * i + 4 * g + e;
-        if (m < M) args.C[(int64_t)m * args.ldc + n] = apply_epilogue_f32<EPI>(acc[i][c][e], bv, args.alpha);
+        const int m = m0 + wm + 16 * i + 4 * g + e;
+        if (m < args.M) args.C[(int64_t)m * args.ldc + n] = apply_epilogue_f32<EPI>(acc[i][c][e], bv, args.alpha);
       }
   }
-}
-
-template <class C, int EPI>
-__device__ __forceinline__ void fp32_wave_tile(const GemmF32Args& args, int m0, int n0) {
-  static_assert(C::RB % 2 == 0, "64-row pieces");
-#pragma unroll 1
-  for (int i = 0; i < C::RB / 2; ++i) fp32_wave_rows<C, EPI>(args, m0 + 64 * i, n0);
 }
 
 template <class C, int EPI>
@@ -187,6 +216,7 @@ gemm_f32_split_kernel(GemmF32Args args) {
   constexpr int RB = C::RB, CB = C::CB, KK = C::KK;
   __shared__ __align__(16) char smem[C::kLds];
   __shared__ int counts[C::BM + C::BN];  // nonzero values of the tile's rows and columns in the first steps
+  __shared__ int biggest;
   for (int i = threadIdx.x; i < C::BM + C::BN; i += C::kThreads) counts[i] = 0;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -219,6 +249,10 @@ gemm_f32_split_kernel(GemmF32Args args) {
   }
 
   constexpr int kOct = C::AO + C::BO;
+  auto line_of = [&](int o) {  // the octet's row, or BM + column, within the tile
+    return o < C::AO ? ((int)threadIdx.x + o * C::kThreads) / C::OPR
+                     : C::BM + (wave + (o - C::AO) * C::kWaves) % (C::BN / 64) * 64 + lane;
+  };
   float raw[kOct][8];
   auto load_octet = [&](float (&raw)[kOct][8], int o, int k0) __attribute__((always_inline)) {
     if (o < C::AO) {
@@ -246,9 +280,10 @@ gemm_f32_split_kernel(GemmF32Args args) {
     }
   };
   uint32_t lost = 0;
+  float big = 0.0f;
   auto stage_octet = [&](char* st, int o) __attribute__((always_inline)) {
     u32x4 p[kPlanes];
-    split8(raw[o], p, lost);
+    split8(raw[o], p, lost, big);
     const int at = o < C::AO ? la[o] : lb[o - C::AO];
 #pragma unroll
     for (int q = 0; q < kPlanes; ++q) *reinterpret_cast<u32x4*>(st + at + q * C::kFrag) = p[q];
@@ -289,9 +324,7 @@ gemm_f32_split_kernel(GemmF32Args args) {
     for (int c = 0; c < kCheck; ++c)
 #pragma unroll
       for (int e = 0; e < 8; ++e) n += first[c][o][e] != 0.0f;
-    const int idx = o < C::AO ? ((int)threadIdx.x + o * C::kThreads) / C::OPR
-                              : C::BM + (wave + (o - C::AO) * C::kWaves) % (C::BN / 64) * 64 + lane;
-    atomicAdd(&counts[idx], n);
+    atomicAdd(&counts[line_of(o)], n);
   }
   __syncthreads();
   bool sparse = full < kCheck;  // its last step has been counted more than once
@@ -322,6 +355,29 @@ gemm_f32_split_kernel(GemmF32Args args) {
   static_assert(kSlices % 2 == 0, "A sets alternate by slice");
   read_a(smem, 0, 0);
   read_b(smem, 0, 0);
+  // Leaves a zero in `counts` only for rows and columns that are zero throughout.
+  auto count_zero_lines = [&] {
+    for (int r = wave; r < C::BM; r += C::kWaves) {
+      if (counts[r] != 0) continue;  // uniform
+      const float* p = args.A + (int64_t)min(m0 + r, M - 1) * args.lda;
+      uint32_t any = 0;
+#pragma unroll 8
+      for (int k = 4 * lane; k < K; k += 256) {
+        const f32x4u v = *reinterpret_cast<const f32x4u*>(p + min(k, K - 4));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) any |= __builtin_bit_cast(uint32_t, v[e]);
+      }
+      if (any & 0x7fffffffu) counts[r] = 1;
+    }
+    for (int c = 0; c < C::BN; c += 64) {
+      if (!__any(counts[C::BM + c + lane] == 0)) continue;  // uniform
+      const float* p = args.B + min(n0 + c + lane, N - 1);
+      uint32_t any = 0;
+#pragma unroll 8
+      for (int k = wave; k < K; k += C::kWaves) any |= __builtin_bit_cast(uint32_t, p[(int64_t)k * args.ldb]);
+      if (any & 0x7fffffffu) counts[C::BM + c + lane] = 1;
+    }
+  };
   // The K loop on PRODUCTS (6 or 8) products and the stores; false, with nothing
   // stored, if the tile must be recomputed.
   auto compute = [&](auto products_c) __attribute__((always_inline)) {
@@ -362,7 +418,7 @@ gemm_f32_split_kernel(GemmF32Args args) {
             load_octet(raw, o, k2);
           }
         }
-        // One MFMA, at most one LDS read, five VALU operations, and so on: the
+        // One MFMA, at most one LDS read, some VALU operations, and so on: the
         // compiler otherwise puts the splitting after the MFMAs.
         constexpr int kReads[2] = {3, 3 + 3 * CB};
         const int reads = kReads[sl == kSlices - 1 || (i == 0 && kk + 1 < KK)];
@@ -370,7 +426,7 @@ gemm_f32_split_kernel(GemmF32Args args) {
         for (int m = 0; m < PRODUCTS * CB; ++m) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
           if (m < reads) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, C::kValu, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -386,14 +442,45 @@ gemm_f32_split_kernel(GemmF32Args args) {
     for (int i = 0; i < RB; ++i)
 #pragma unroll
       for (int j = 0; j < CB; ++j) acc[i][j] += low[i][j];
-    bool bad = (lost & 0xffffu) != 0;
+    // `zero` turns NaN if a sum is not finite.
+    float zero = 0.0f, least = __builtin_huge_valf();
 #pragma unroll
     for (int i = 0; i < RB; ++i)
 #pragma unroll
       for (int j = 0; j < CB; ++j)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) bad |= !(__builtin_fabsf(acc[i][j][e]) < __builtin_huge_valf());
-    if (__syncthreads_or(bad)) return false;  // uniform
+        for (int e = 0; e < 16; ++e) {
+          zero = __builtin_fmaf(acc[i][j][e], 0.0f, zero);
+          least = __builtin_fminf(least, __builtin_fabsf(acc[i][j][e]));
+        }
+    const float underflow = 0x1p-124f * (float)K;
+    const bool cut = (lost & 0xffffu) != 0;
+    if (__syncthreads_or(zero != 0.0f || least < underflow || cut)) {  // uniform
+      if (threadIdx.x == 0) biggest = 0;
+      __syncthreads();
+      atomicMax(&biggest, __builtin_bit_cast(int, big));
+      const bool any_cut = __syncthreads_or(cut);
+      float limit = underflow;
+      if (any_cut) {
+        limit = fmaxf(limit, 0x1.02p-105f * (float)K * __builtin_bit_cast(float, biggest));
+        count_zero_lines();
+        __syncthreads();
+      }
+      bool bad = zero != 0.0f;
+#pragma unroll
+      for (int j = 0; j < CB; ++j) {
+        const bool col = any_cut & (counts[C::BM + (wn * CB + j) * 32 + (lane & 31)] != 0);
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const int row = counts[(wm * RB + i) * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3)];
+            const float v = __builtin_fabsf(acc[i][j][e]);
+            bad |= (v < limit) & ((v != 0.0f) | (col & (row != 0)));
+          }
+      }
+      if (__syncthreads_or(bad)) return false;
+    }
     // Lane: rows 8 (r/4) + 4 (lane/32) + r%4 and column lane%32 of a block, so
     // each store writes two 128-byte row segments. The stores go through a
     // descriptor of C's rows m0 .. M-1, whose range check drops rows past M;
@@ -421,7 +508,16 @@ gemm_f32_split_kernel(GemmF32Args args) {
     return true;
   };
   const bool done = eight ? compute(std::integral_constant<int, 8>{}) : compute(std::integral_constant<int, 6>{});
-  if (!done) fp32_wave_tile<C, EPI>(args, m0 + wm * RB * 32, n0 + wn * CB * 32);
+  if (done) return;
+  fp32_tile<C, EPI>(args, smem, m0, n0, nit, raw, [&](int it) __attribute__((always_inline)) {
+    if (it == 0 && has_tail) {
+#pragma unroll
+      for (int o = 0; o < kOct; ++o) load_tail(o, full * C::BK);
+    } else {
+#pragma unroll
+      for (int o = 0; o < kOct; ++o) load_octet(raw, o, k_of(it));
+    }
+  });
 }
 
 template <class C>
@@ -451,9 +547,9 @@ hipError_t launch_tile(int epi, GemmF32Args a, hipStream_t stream) {
 hipError_t launch_gemm_f32_split(int tile, int epi, GemmF32Args a, hipStream_t stream) {
   if (a.M < 1 || a.N < 1 || a.K < 32 || a.ldc >= kF32SplitMaxLdc) return hipErrorInvalidValue;  // a full step of K
   switch (tile) {
-    case kSplit256x128: return launch_tile<SplitTile<256, 128, 2, 2, 16, 1>>(epi, a, stream);
-    case kSplit128W8: return launch_tile<SplitTile<128, 128, 2, 4, 32, 2>>(epi, a, stream);
-    case kSplit128Pair: return launch_tile<SplitTile<128, 128, 2, 2, 16, 2>>(epi, a, stream);
+    case kSplit256x128: return launch_tile<SplitTile<256, 128, 2, 2, 16, 1, 5>>(epi, a, stream);
+    case kSplit128W8: return launch_tile<SplitTile<128, 128, 2, 4, 32, 2, 8>>(epi, a, stream);
+    case kSplit128Pair: return launch_tile<SplitTile<128, 128, 2, 2, 16, 2, 8>>(epi, a, stream);
     default: return hipErrorInvalidValue;
   }
 }
