@@ -208,11 +208,14 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
       it = itn;
     };
     int i = 1;
-    for (; i + 1 < nit; i += 2) {
-      iteration(std::integral_constant<int, 0>{});
-      iteration(std::integral_constant<int, kU % 2>{});
-    }
-    if (i < nit) iteration(std::integral_constant<int, 0>{});
+    // Unrolled only where the sets swap from one iteration to the next
+    // (48x4096x4097 with one set 25.4 -> 24.7 us, 48x8192x8192 63.9 -> 62.2).
+    if constexpr (NS > 1 && kU % 2 != 0)
+      for (; i + 1 < nit; i += 2) {
+        iteration(std::integral_constant<int, 0>{});
+        iteration(std::integral_constant<int, 1>{});
+      }
+    for (; i < nit; ++i) iteration(std::integral_constant<int, 0>{});
 #pragma unroll
     for (int q = 0; q < 4 * kU; ++q) mfma_q(sum[(1 - q / 4) % NS], x[q / 4], q % 4, w[q]);
   }
@@ -317,17 +320,19 @@ gemv_f32_kernel(GemvF32Args a, int epi) {
 // All split loads are issued before the first add so their latencies overlap.
 // W, the bias and Y may have any alignment; the last four columns of a row
 // that N cuts short are read and written one by one. The partials always have
-// an aligned row pitch (ldp, a multiple of 4).
+// an aligned row pitch (ldp, a multiple of 4). FULL: N % 4 == 0, no such columns
+// (no load then waits behind a branch: 33x1235x1408 11.2 -> 10.9 us).
 // One wave per workgroup spreads the reduction over more CUs than 256-thread
 // workgroups (the c4 column shard: 16 workgroups of 256 threads); measured
 // 0.2 us faster per layer at c4 and at its column shard.
+template <bool FULL>
 __global__ void __launch_bounds__(64) gemv_reduce_kernel(GemvF32Args a, int epi, int prow) {
   const int64_t idx = (int64_t)blockIdx.x * 64 + threadIdx.x;  // over M * ceil(N/4)
   const int n4 = (a.N + 3) / 4;
   if (idx >= (int64_t)a.M * n4) return;
   const int row = (int)(idx / n4);
   const int col = 4 * (int)(idx % n4);
-  const bool full = col + 4 <= a.N;
+  const bool full = FULL || col + 4 <= a.N;
   f32x4 v[kMaxSplit];
 #pragma unroll
   for (int sp = 0; sp < kMaxSplit; ++sp)
@@ -442,7 +447,10 @@ hipError_t launch_gemv_f32(int epi, int cols, GemvF32Args a, hipStream_t stream)
   if (e != hipSuccess || a.ksplit == 1) return e;
   const int64_t items = (int64_t)a.M * ((a.N + 3) / 4);
   const dim3 g((unsigned)((items + 63) / 64));
-  hipLaunchKernelGGL(gemv_reduce_kernel, g, dim3(64), 0, stream, a, epi, 16 * mb);
+  if (a.N % 4 == 0)
+    hipLaunchKernelGGL(gemv_reduce_kernel<true>, g, dim3(64), 0, stream, a, epi, 16 * mb);
+  else
+    hipLaunchKernelGGL(gemv_reduce_kernel<false>, g, dim3(64), 0, stream, a, epi, 16 * mb);
   return hipGetLastError();
 }
 
