@@ -1,5 +1,5 @@
 // fp32 dense layer / matmul for small outputs, any shape, row stride and
-// alignment: a 16x16 tile per workgroup of 4, 8 or 16 waves that split K.
+// alignment: a 16x16 tile per workgroup of 4 or 8 waves that split K.
 //
 // C[M,N] = epilogue(A[M,K] x B[K,N] (+ bias[N])) -- the same op as the other
 // tiles (reference cpp/src/builders/LinalgBuilder.cpp:106-139, 180-239,
@@ -125,7 +125,6 @@ hipError_t launch_gemm_f32_small(int waves, int epi, GemmF32Args a, hipStream_t 
   switch (waves) {
     case 4: hipLaunchKernelGGL(gemm_f32_small_kernel<4>, grid, block, 0, stream, a, epi); break;
     case 8: hipLaunchKernelGGL(gemm_f32_small_kernel<8>, grid, block, 0, stream, a, epi); break;
-    case 16: hipLaunchKernelGGL(gemm_f32_small_kernel<16>, grid, block, 0, stream, a, epi); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

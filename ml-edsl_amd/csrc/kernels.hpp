@@ -53,7 +53,7 @@ hipError_t launch_gemm_f32_direct_rc(int r, int c, int guard, int epi, GemmF32Ar
 // The tiles on bf16 matrix cores at fp32 precision (gemm_f32_split.hip), `tile`
 // an F32SplitTile: any M, N, alignment and row strides, K >= 32.
 hipError_t launch_gemm_f32_split(int tile, int epi, GemmF32Args args, hipStream_t stream);
-// 16x16 tiles for small outputs (gemm_f32_small.hip), K split over 4, 8 or 16
+// 16x16 tiles for small outputs (gemm_f32_small.hip), K split over 4 or 8
 // waves of a workgroup: any M, N, K >= 1, alignment and row strides.
 hipError_t launch_gemm_f32_small(int waves, int epi, GemmF32Args args, hipStream_t stream);
 
