@@ -91,13 +91,14 @@ int edsl_hip_dense_i32_launch(const int32_t *X, int64_t ldx, const int32_t *W, i
 
 /* Description of the kernels the calling thread's last call launched, e.g.
  * "gemm_f32 cfg=f32_256x256x16_w4x4 grid=256" (a "_edge" suffix: partial
- * edge tiles), "gemm_f32 split=bf16x6 tile=... grid=256 in place of cfg=..."
- * (the bf16 matrix cores at fp32 precision, and the fp32 tile they replace),
- * "gemv_f32 mb=1 ksplit=4 cols=128 grid=256 +reduce" (with
- * "+xunaligned", "+wrealigned", "+wunaligned": rows of X or W that are not
- * 16-byte aligned; "+ktail": K % 16 rows apart from the 16-deep
- * steps; "tile=16x16": a small layer in one launch, K split over the waves of
- * a workgroup), "narrow_i8+gemm_i8 variant=3 waves=ksplit depth=2 grid=256"
+ * edge tiles), "gemm_f32 split=bf16x6 tile=256x128x16 grid=512" (the bf16
+ * matrix cores at fp32 precision), "gemm_f32_small tile=16x16 waves=4 grid=64"
+ * (K split over the waves of a workgroup),
+ * "gemv_f32 mb=1 ksplit=4 cols=128 grid=256 +reduce" (with "+xunaligned": rows
+ * of X that are not 16-byte aligned; "+wshared": rows of W that do not start on
+ * 128-byte lines, read through the caches; "+wscalar": N < 4; "+ktail": K % 16
+ * rows apart from the 16-deep steps),
+ * "narrow_i8+gemm_i8 variant=3 waves=ksplit depth=2 grid=256"
  * or "narrow_i8+gemm_i8 tile=64x64 waves=ksplit grid=128"; returns its length. */
 int edsl_hip_last_plan(char *buf, size_t len);
 

@@ -435,12 +435,7 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
   const int waves = tuned_small_m ? 0 : plan_f32_small(query, stream_rows);
   if (waves > 0) {
     check_hip(launch_gemm_f32_small(waves, L.epi, t, stream), "gemm_f32_small launch");
-    const int grid = ((M + 15) / 16) * ((N + 15) / 16);
-    if (M <= kGemvMaxM && (small_m || !w_vec))
-      set_plan("gemv_f32 mb=%d ksplit=%d cols=16 tile=16x16 grid=%d%s%s%s", row_blocks, waves, grid,
-               x_vec ? "" : " +xunaligned", w_vec ? "" : " +wunaligned", K % 16 ? " +ktail" : "");
-    else
-      set_plan("gemm_f32 cfg=f32_16x16_anyshape_k%d grid=%d", waves, grid);
+    set_plan("gemm_f32_small tile=16x16 waves=%d grid=%d", waves, ((M + 15) / 16) * ((N + 15) / 16));
     return;
   }
 
@@ -494,7 +489,7 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
     set_plan("gemv_f32 mb=%d ksplit=%d cols=%d grid=%d%s%s%s%s%s", mb, a.ksplit, gemv_cols,
              ((N + gemv_cols - 1) / gemv_cols) * a.ksplit, a.ksplit > 1 ? " +reduce" : "",
              x_vec ? "" : " +xunaligned",
-             w_vec ? "" : N >= 4 && gemv_cols > 32 ? " +wrealigned" : " +wunaligned", tail ? " +ktail" : "",
+             a.w_mode == kWVector ? "" : a.w_mode == kWShared ? " +wshared" : " +wscalar", tail ? " +ktail" : "",
              fixed && scratch ? " +fixed-scratch" : "");
     return;
   }
@@ -509,8 +504,7 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
   const int split = plan_f32_split(query, cfg);
   if (split != kSplitNone) {
     check_hip(launch_gemm_f32_split(split, L.epi, t, stream), "gemm_f32_split launch");
-    set_plan("gemm_f32 split=bf16x6 tile=%s grid=%lld in place of cfg=%s grid=%d", f32_split_name(split),
-             (long long)f32_split_grid(split, M, N), g.name, t.tiles_m * t.tiles_n);
+    set_plan("gemm_f32 split=bf16x6 tile=%s grid=%lld", f32_split_name(split), (long long)f32_split_grid(split, M, N));
     return;
   }
   check_hip(launch_gemm_f32(cfg, L.epi, t, stream), "gemm_f32 launch");

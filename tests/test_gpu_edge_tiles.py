@@ -3,10 +3,10 @@
 The fp32 tiles have edge variants (partial tiles at the M, N and K edges,
 16-byte vector loads at clamped addresses, masked stores) for 16-byte aligned
 operands whose K, N and row strides are multiples of 4, and any-shape variants
-(element-checked 4-byte loads and stores) for every other layout; the small-M kernel
-spreads K over its wave slices in 16-row chunks, so K need only be a multiple
-of 16, and its last column block may be partial, so N need only be a multiple
-of 4. Every case is checked against the oracle on the full output.
+(element-checked 4-byte loads and stores) for every other layout; the small-M
+kernel spreads K over its wave slices in 16-row chunks, the K % 16 rows apart,
+and its last column block may be partial. Every case is checked against the
+oracle on the full output.
 """
 from __future__ import annotations
 
@@ -80,27 +80,50 @@ def test_every_edge_config_on_odd_shapes(torch_cuda):
         set_f32_config(-1)
 
 
-@pytest.mark.parametrize("shape, tile", [
-    ((1000, 1000, 1000), "f32_64x64x64_direct_k4_edge"),
-    ((4000, 256, 4000), "f32_128x128x16_direct_edge"),
-    # 33 x 32 tiles of 128x128 would give 32 CUs a fifth tile
-    ((4097, 256, 4096), "f32_64x64x64_mfma16_edge"),
-    # K = 1000 leaves a partial last K step on every tile
-    ((512, 1000, 512), "f32_32x32x64_direct_rc_edge"),
-], ids=["1000^3", "4000x256x4000", "4097x256x4096", "512x1000x512"])
-def test_auto_plan_takes_edge_tiles(shape, tile, torch_cuda):
-    M, K, N = shape
+def _check_auto_plan(torch, M, K, N, tile, split, pad=0, off=0):
+    """The automatic plan takes `tile`, or, where the layer runs on the bf16
+    matrix cores, `split`; the fp32 tile is then run forced."""
+    from mlir_edsl_hip.device import set_f32_config
     X, W, b = _inputs(M, K, N, M + K + N)
-    got, plan = _run(torch_cuda, X, W, b)
-    assert f"cfg={tile} " in plan, plan
-    assert_f32_parity(got, oracle.dense_f32_chains(X, W, b, "relu"), K)
+    ref = oracle.dense_f32_chains(X, W, b, "relu")
+    got, plan = _run(torch, X, W, b, pad, off)
+    assert plan.startswith(f"gemm_f32 split=bf16x6 tile={split} " if split else f"gemm_f32 cfg={tile} "), plan
+    assert_f32_parity(got, ref, K)
+    if split:
+        try:
+            set_f32_config(_native.f32_config_names().index(tile))
+            got, plan = _run(torch, X, W, b, pad, off)
+        finally:
+            set_f32_config(-1)
+        assert plan.startswith(f"gemm_f32 cfg={tile} "), plan
+        assert_f32_parity(got, ref, K)
+
+
+@pytest.mark.parametrize("shape, tile, split", [
+    ((1000, 1000, 1000), "f32_64x64x64_direct_k4_edge", None),
+    ((4000, 256, 4000), "f32_128x128x16_direct_edge", "128x128x16"),
+    ((4000, 252, 4000), "f32_128x128x16_direct_edge", None),
+    # 33 x 32 tiles of 128x128 would give 32 CUs a fifth tile
+    ((4097, 256, 4096), "f32_64x64x64_mfma16_edge", "128x128x16"),
+    ((4097, 252, 4096), "f32_64x64x64_mfma16_edge", None),
+    # K = 1000 leaves a partial last K step on every tile
+    ((512, 1000, 512), "f32_32x32x64_direct_rc_edge", None),
+], ids=["1000^3", "4000x256x4000", "4000x252x4000", "4097x256x4096", "4097x252x4096", "512x1000x512"])
+def test_auto_plan_takes_edge_tiles(shape, tile, split, torch_cuda):
+    _check_auto_plan(torch_cuda, *shape, tile, split)
+
+
+@pytest.mark.parametrize("shape, tile, split", [((2048, 2048, 2048), "f32_64x64x16_direct", "128x128x32_w8"),
+                                                ((4096, 1024, 4096), "f32_128x128x16_direct", "256x128x16")],
+                         ids=["2048^3", "4096x1024x4096"])
+def test_aligned_shapes_on_the_bf16_matrix_cores(shape, tile, split, torch_cuda):
+    _check_auto_plan(torch_cuda, *shape, tile, split)
 
 
 def test_aligned_shapes_keep_their_tiles(torch_cuda):
     """Shapes the tiles divide still take the unguarded configurations."""
     for (M, K, N), tile in (((1024, 1024, 1024), "f32_64x64x64_direct_rc"),
-                            ((2048, 2048, 2048), "f32_64x64x16_direct"),
-                            ((4096, 1024, 4096), "f32_128x128x16_direct"),
+                            ((4096, 240, 4096), "f32_128x128x16_direct"),
                             ((3072, 512, 3072), "f32_64x64x64_direct_k4"),
                             ((2048, 128, 2048), "f32_128x128x32_mfma16_w8"),
                             ((1024, 128, 1024), "f32_64x64x64_mfma16"),
@@ -114,11 +137,13 @@ def test_aligned_shapes_keep_their_tiles(torch_cuda):
         assert_f32_parity(got, oracle.dense_f32_chains(X, W, b, "relu"), K)
 
 
-def test_unaligned_k_takes_an_any_shape_tile(torch_cuda):
-    """K not a multiple of 4 leaves rows unaligned: an element-checked tile."""
-    X, W, b = _inputs(70, 37, 50, 9)
+@pytest.mark.parametrize("M, N, kernel", [(70, 50, "gemm_f32_small "), (700, 1001, "gemm_f32 cfg=f32_32x32x64")])
+def test_unaligned_k_takes_an_any_shape_tile(M, N, kernel, torch_cuda):
+    """K not a multiple of 4 leaves rows unaligned: the 16x16 tiles, or an
+    element-checked tile."""
+    X, W, b = _inputs(M, 37, N, 9)
     got, plan = _run(torch_cuda, X, W, b)
-    assert "anyshape" in plan, plan
+    assert plan.startswith(kernel) and ("tile=16x16" in plan or "anyshape" in plan), plan
     assert_f32_parity(got, oracle.dense_f32_chains(X, W, b, "relu"), 37)
 
 
@@ -146,19 +171,18 @@ def test_every_any_shape_config_on_odd_shapes(torch_cuda):
         set_f32_config(-1)
 
 
-@pytest.mark.parametrize("shape, pad_off, tile", [
-    ((2001, 2001, 2001), (0, 0), "f32_128x128x32_mfma16_anyshape"),
-    ((1025, 1025, 1025), (0, 0), "f32_64x64x64_w2x2_k2_pf2_anyshape"),
+@pytest.mark.parametrize("shape, pad_off, tile, split", [
+    ((2001, 2001, 2001), (0, 0), "f32_128x128x32_mfma16_anyshape", "128x128x32_w8"),
+    ((2001, 251, 2001), (0, 0), "f32_128x128x32_mfma16_anyshape", None),
+    ((1025, 1025, 1025), (0, 0), "f32_64x64x64_w2x2_k2_pf2_anyshape", None),
     # K = N = 2048 but every row misaligned by an element offset
-    ((2048, 2048, 2048), (0, 1), "f32_128x128x32_mfma16_anyshape"),
-    ((4001, 1001, 4001), (0, 0), "f32_256x256x16_w4x4_anyshape"),
-], ids=["2001^3", "1025^3", "2048^3-offset", "4001x1001x4001"])
-def test_auto_plan_takes_any_shape_tiles(shape, pad_off, tile, torch_cuda):
-    M, K, N = shape
-    X, W, b = _inputs(M, K, N, M + 3 * K + N)
-    got, plan = _run(torch_cuda, X, W, b, *pad_off)
-    assert f"cfg={tile} " in plan, plan
-    assert_f32_parity(got, oracle.dense_f32_chains(X, W, b, "relu"), K)
+    ((2048, 2048, 2048), (0, 1), "f32_128x128x32_mfma16_anyshape", "128x128x32_w8"),
+    ((2048, 240, 2048), (0, 1), "f32_128x128x32_mfma16_anyshape", None),
+    ((4001, 1001, 4001), (0, 0), "f32_256x256x16_w4x4_anyshape", "256x128x16"),
+    ((4001, 251, 4001), (0, 0), "f32_256x256x16_w4x4_anyshape", None),
+], ids=["2001^3", "2001x251x2001", "1025^3", "2048^3-offset", "2048x240x2048-offset", "4001x1001x4001", "4001x251x4001"])
+def test_auto_plan_takes_any_shape_tiles(shape, pad_off, tile, split, torch_cuda):
+    _check_auto_plan(torch_cuda, *shape, tile, split, *pad_off)
 
 
 def _run_small_m(torch, X, W, b, pad=0, off=0):
@@ -181,24 +205,23 @@ def test_small_m_uneven_k_slices(M, K, N, torch_cuda):
 
 
 # Small M with W, Y and bias rows that are not 16-byte aligned or N not a
-# multiple of 4: W realigned from two 16-byte chunks per row (N >= 4, four
-# columns per lane) or read per column, Y and the bias per element, columns
-# past N never stored; the last row of W and any odd K go through the reduce
-# kernel's tail. One to four row blocks, each column width the plan picks,
-# contiguous and misaligned views (pad 0 puts W's last element at the end of
-# its buffer).
+# multiple of 4: W read with one vector load per lane and row at any alignment,
+# or (N < 4) per column; columns past N never stored; any K % 16 rows go
+# through the reduce kernel's tail. One to four row blocks, each column width
+# the plan picks, contiguous and misaligned views (pad 0 puts W's last element
+# at the end of its buffer).
 @pytest.mark.parametrize("M, K, N", [(16, 8192, 8191), (16, 4096, 5003), (5, 1003, 1029), (64, 2048, 1023),
                                      (33, 512, 7), (1, 512, 3), (48, 4096, 4097)])
 def test_small_m_unaligned_w(M, K, N, torch_cuda):
-    """The automatic plan (the small-M kernel or the 32x32 any-shape tile,
-    whichever measured faster for the shape), then the small-M kernel itself
-    under a forced split of 2."""
+    """The automatic plan (the small-M kernel, the 16x16 tiles or the 32x32
+    any-shape tile, whichever measured faster for the shape), then the small-M
+    kernel itself under a forced split of 2."""
     from mlir_edsl_hip.device import set_gemv_ksplit
     X, W, b = _inputs(M, K, N, M * 7 + K + N)
     ref = oracle.dense_f32_chains(X, W, b, "relu")
     for pad, off in ((0, 0), (3, 1)):
         got, plan = _run(torch_cuda, X, W, b, pad, off)
-        assert "+wunaligned" in plan or "+wrealigned" in plan or "32x32x64" in plan, plan
+        assert plan.startswith(("gemv_f32 ", "gemm_f32_small ")) or "32x32x64" in plan, plan
         assert_f32_parity(got, ref, K)
         try:
             set_gemv_ksplit(2)
@@ -206,17 +229,17 @@ def test_small_m_unaligned_w(M, K, N, torch_cuda):
         finally:
             set_gemv_ksplit(0)
         assert plan.startswith("gemv_f32") and "ksplit=2" in plan, plan
-        assert ("+wrealigned" if N >= 4 and "cols=32 " not in plan else "+wunaligned") in plan, plan
+        assert ("+wshared" if N >= 4 else "+wscalar") in plan, plan
         assert_f32_parity(got, ref, K)
 
 
-# Realigned W rows at every offset of a row within its 16-byte chunk: row
-# pitches N + pad and element offsets chosen so that the offset of row k
-# cycles with k when the pitch is odd; N such that the last lane of a lane
-# group (the one that loads its own second chunk) holds a column below N,
-# straddles N or lies past it, on every column width; one to three row blocks
-# (second chunk from the neighbouring lane) and four (both chunks loaded by
-# every lane). K = 1029: the last rows, the last one always, go to the tail.
+# W rows at every offset within 16 bytes, each read with one vector load per
+# lane: row pitches N + pad and element offsets chosen so that the offset of
+# row k cycles with k when the pitch is odd; N such that the last lane of a
+# lane group holds a column below N, straddles N (it then loads the last four
+# columns) or lies past it, on every column width; one to four row blocks. K =
+# 1029: the last rows go to the tail. Rows that all start on 128-byte lines are
+# streamed past the caches, the others read through them.
 @pytest.mark.parametrize("cols", [64, 128, 256])
 @pytest.mark.parametrize("M", [1, 17, 40, 64])
 def test_realigned_w_rows(M, cols, torch_cuda):
@@ -235,9 +258,9 @@ def test_realigned_w_rows(M, cols, torch_cuda):
                 set_gemv_ksplit(0)
                 set_gemv_cols(0)
             what = f"M={M} K={K} N={N} pad={pad} off={off} [{plan}]"
-            vector_rows = N % 4 == 0 and pad % 4 == 0 and off % 4 == 0
+            streamed = (N + pad) % 32 == 0 and off % 32 == 0
             assert plan.startswith("gemv_f32") and f"cols={cols} " in plan, what
-            assert ("+wrealigned" in plan) != vector_rows, what
+            assert ("+wshared" in plan) != streamed, what
             try:
                 assert_f32_parity(got, ref, K)
             except AssertionError as e:
@@ -248,12 +271,14 @@ def test_realigned_w_rows(M, cols, torch_cuda):
 
 # The automatic choice between the small-M kernel and the tiles for aligned
 # operands: short K goes to the tiles (32x32 tiles read W once up to 32 rows,
-# twice up to 64), long K to the small-M kernel.
+# twice up to 64; 16x16 tiles up to K = 1024 where there are few of them), long
+# K to the small-M kernel.
 @pytest.mark.parametrize("M, K, N, kernel", [
-    (16, 512, 512, "gemv_f32"), (1, 256, 256, "gemm_f32"), (16, 256, 4096, "gemm_f32"),
-    (32, 2048, 1024, "gemv_f32"), (32, 512, 512, "gemm_f32"), (48, 2048, 2048, "gemv_f32"),
-    (48, 1024, 4096, "gemm_f32"), (64, 256, 256, "gemm_f32"), (64, 4096, 1024, "gemv_f32"),
-    (64, 4096, 8192, "gemv_f32"), (64, 2048, 8192, "gemm_f32"), (64, 2048, 2048, "gemm_f32"),
+    (16, 512, 512, "gemm_f32_small "), (1, 256, 256, "gemm_f32_small "), (16, 256, 4096, "gemm_f32_small "),
+    (16, 1040, 512, "gemv_f32 "), (16, 1024, 16384, "gemv_f32 "),
+    (32, 2048, 1024, "gemv_f32 "), (32, 512, 512, "gemm_f32_small "), (48, 2048, 2048, "gemv_f32 "),
+    (48, 1024, 4096, "gemm_f32 "), (64, 256, 256, "gemm_f32_small "), (64, 4096, 1024, "gemv_f32 "),
+    (64, 4096, 8192, "gemv_f32 "), (64, 2048, 8192, "gemm_f32 "), (64, 2048, 2048, "gemm_f32 "),
 ])
 def test_auto_choice_small_m_or_tile(M, K, N, kernel, torch_cuda):
     X, W, b = _inputs(M, K, N, M + 5 * K + N)
@@ -332,7 +357,7 @@ def _run_x_view(torch, X, W, b, x_pad, x_off, ksplit=None, epi=_native.EPI_BIAS_
     (16, 8191, 8192, 0, 0, ("+xunaligned", "+ktail")),   # contiguous X, odd K: unaligned rows
     (16, 8192, 2048, 0, 1, ("+xunaligned",)),             # misaligned X base, K % 16 == 0
     (33, 4100, 512, 0, 0, ("+ktail",)),                   # aligned X, K % 16 == 4
-    (5, 1003, 1024, 2, 3, ("+xunaligned", "+ktail")),
+    (5, 1035, 1024, 2, 3, ("+xunaligned", "+ktail")),
 ], ids=["odd-K", "misaligned-X", "aligned-tail", "both"])
 def test_small_m_k_tail_and_unaligned_x(M, K, N, x_pad, x_off, tags, torch_cuda):
     X, W, b = _inputs(M, K, N, M + K + N)
@@ -351,12 +376,11 @@ _TAIL_EPIS = {"none": (_native.EPI_NONE, None, "none"), "bias": (_native.EPI_BIA
 
 @pytest.mark.parametrize("epi_name", sorted(_TAIL_EPIS))
 @pytest.mark.parametrize("M", [1, 32, 64])
-@pytest.mark.parametrize("K, x_pad, x_off", [(2047, 0, 0), (4099, 3, 1), (1003, 0, 2)],
+@pytest.mark.parametrize("K, x_pad, x_off", [(2047, 0, 0), (4099, 3, 1), (1035, 0, 2)],
                          ids=["odd-K", "padded-offset", "offset"])
 def test_small_m_tail_and_unaligned_x_per_row_block_and_epilogue(M, K, x_pad, x_off, epi_name, torch_cuda):
-    """Unaligned X rows (read with 4-byte loads) and the K tail for one, two
-    and four row blocks, with every epilogue the reduce kernel applies after
-    adding the tail."""
+    """Unaligned X rows and the K tail for one, two and four row blocks, with
+    every epilogue the reduce kernel applies after adding the tail."""
     epi, use_b, act = _TAIL_EPIS[epi_name]
     N = 1024
     X, W, b = _inputs(M, K, N, 7 * M + K)
@@ -380,7 +404,7 @@ def test_single_row_x_with_any_row_stride(K, torch_cuda):
     tY = torch_cuda.full((1, N), float("nan"), device="cuda")
     dense_launch(tX, tW, tb, tY, _native.EPI_BIAS_RELU)
     torch_cuda.cuda.synchronize()
-    assert _native.last_plan().startswith("gemv_f32"), _native.last_plan()
+    assert _native.last_plan().startswith("gemm_f32_small " if K <= 1024 else "gemv_f32 "), _native.last_plan()
     assert_f32_parity(tY.cpu().numpy(), oracle.dense_f32_chains(X, W, b, "relu"), K)
     # Row stride 0 through the C ABI directly (torch reports the view's own
     # stride; a broadcast (1, K) row from expand() has stride 0 on dim 0).
@@ -440,8 +464,8 @@ def test_int8_path_on_odd_shapes(M, K, N, torch_cuda):
 
 def test_int8_path_odd_shapes_strided_and_out_of_range(torch_cuda):
     """Padded, offset device views (the narrowing pass's unaligned loads on
-    edge tiles), then a value outside int8 (the exact i32 fallback on the
-    original tensors), then in range again."""
+    edge tiles), then a value outside int8 (a second digit plane), then in range
+    again."""
     from mlir_edsl_hip.device import dense_launch
     M, K, N = 300, 250, 190
     rng = np.random.default_rng(21)

@@ -244,8 +244,8 @@ def test_int8_path_falls_back_when_values_leave_int8(torch_cuda):
 
 def test_int8_fallback_is_per_tile(torch_cuda):
     """Values outside int8 in a few 64x64 tiles of X and W: the tiles whose
-    panels hold them take the exact i32 path, the others the int8 path, and
-    every output is exact, for every variant."""
+    panels hold them run the products of several digit planes, the others one
+    product, and every output is exact, for every variant."""
     from mlir_edsl_hip.device import set_i8_variant
     rng = np.random.default_rng(16)
     M, K, N = 640, 768, 896
@@ -275,7 +275,7 @@ def test_every_int8_variant(torch_cuda):
     W = rng.integers(-128, 128, size=(K, N), dtype=np.int32)
     b = rng.integers(-2**20, 2**20, size=(N,), dtype=np.int32)
     Xbig = X.copy()
-    Xbig[5, 7] = 1000  # forces the exact i32 fallback inside the same kernel
+    Xbig[5, 7] = 1000  # a second digit plane for the tiles of its row panel
     n = _native.lib().edsl_hip_i8_variant_count()
     try:
         for v in range(n):

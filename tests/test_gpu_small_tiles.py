@@ -44,7 +44,7 @@ def test_small_tiles(M, K, N, pad, off):
         dense_launch(tX, tW, tb if has_bias else None, tY, epi, 0.125)
         torch.cuda.synchronize()
         plan = _native.last_plan()
-        assert "tile=16x16" in plan or "cfg=f32_16x16_anyshape" in plan, plan
+        assert plan.startswith("gemm_f32_small tile=16x16 "), plan
         assert_f32_parity(tY.cpu().numpy(), oracle.dense_f32_chains(X, W, b if has_bias else None, act, 0.125), K)
         tY.fill_(7.0)
         assert (ybuf == 7.0).all()  # nothing else was written
