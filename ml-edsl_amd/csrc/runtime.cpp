@@ -29,6 +29,7 @@
 #include "../../include/edsl_hip.h"
 #include "../../include/edsl_hip_device.h"
 #include "common.hpp"
+#include "dev_buf.hpp"
 #include "kernels.hpp"
 #include "host_stage.hpp"
 #include "runtime_internal.hpp"
@@ -73,47 +74,6 @@ int copy_out(const std::string& s, char* buf, size_t len) {
 }
 
 // ------------------------------------------------------------ device state
-struct DevBuf {
-  void* p = nullptr;
-  size_t cap = 0;
-  // Workspaces of the device entry points may be baked into HIP graphs that
-  // callers capture, so an outgrown one is kept (retired) rather than freed:
-  // a replay still finds the buffer it was captured with. Growth is then at
-  // least twofold, which bounds the retired total by the final capacity.
-  bool keep_old = false;
-  std::vector<void*> retired;
-
-  DevBuf() = default;
-  explicit DevBuf(bool keep) : keep_old(keep) {}
-
-  // Grow-only. A buffer that is released may still be in use by queued work,
-  // so the device is drained first.
-  void* ensure(size_t bytes, bool zero_fill) {
-    if (bytes <= cap && p) return p;
-    size_t grow = 0;
-    if (p && keep_old) {
-      retired.push_back(p);
-      grow = 2 * cap;
-      p = nullptr;
-      cap = 0;
-    } else if (p) {
-      check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize");
-      check_hip(hipFree(p), "hipFree");
-      p = nullptr;
-      cap = 0;
-    }
-    const size_t want = std::max<size_t>({(bytes + 255) & ~size_t(255), size_t(256), grow});
-    check_hip(hipMalloc(&p, want), "hipMalloc");
-    if (zero_fill) {
-      // Finished before any stream (blocking or not) can use the buffer.
-      check_hip(hipMemset(p, 0, want), "hipMemset");
-      check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize");
-    }
-    cap = want;
-    return p;
-  }
-};
-
 constexpr int kPipeBlocks = 4;  // row blocks of a pipelined host-buffer layer
 
 struct DeviceState {
@@ -482,7 +442,7 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
       if (part_bytes) a.partials = reinterpret_cast<float*>(fixed->base);
     } else if (scratch) {
       scratch_begin(ds, stream);
-      a.partials = static_cast<float*>(ds.gemv_partials.ensure(part_bytes, false));
+      a.partials = static_cast<float*>(ds.gemv_partials.ensure(part_bytes));
     }
     check_hip(launch_gemv_f32(L.epi, gemv_cols, a, stream), "gemv_f32 launch");
     if (scratch && !fixed) scratch_end(ds, stream);
@@ -531,17 +491,25 @@ void launch_i32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream) {
   // outside int8 take several digits). Its packed copies
   // are padded with zeros to multiples of the 128-wide tile, so any M, N and
   // K run on it; only the stores are limited to the real M x N.
-  const bool tiled = a.M > 0 && a.N > 0 && a.K > 0 && a.K < (1 << 17);
+  bool tiled = a.M > 0 && a.N > 0 && a.K > 0 && a.K < (1 << 17);
+  auto pad = [](int v) { return (v + kI8Tile - 1) / kI8Tile * kI8Tile; };
+  const int Mp = pad(a.M), Np = pad(a.N), Kp = pad(a.K);
+  const size_t xs = (size_t)Mp * Kp, ws = (size_t)Np * Kp;
+  // One digit count per 64x64 tile of the padded X and W (rewritten by every call).
+  const size_t fx = (size_t)(Mp / 64) * (Kp / 64), fw = (size_t)(Np / 64) * (Kp / 64);
+  int8_t *x8 = nullptr, *w8 = nullptr;
+  uint8_t* flags = nullptr;
   if (tiled) {
-    auto pad = [](int v) { return (v + kI8Tile - 1) / kI8Tile * kI8Tile; };
-    const int Mp = pad(a.M), Np = pad(a.N), Kp = pad(a.K);
+    // The host does not know how many digits the values need: room for all
+    // planes, the size of X and W themselves. Where the device has not that
+    // much, the vector-ALU kernel, which needs none, takes the layer.
+    x8 = static_cast<int8_t*>(ds.i8_x.try_ensure(kI8Digits * xs));
+    w8 = x8 ? static_cast<int8_t*>(ds.i8_w.try_ensure(kI8Digits * ws)) : nullptr;
+    flags = w8 ? static_cast<uint8_t*>(ds.i8_flags.try_ensure(fx + fw)) : nullptr;
+    tiled = flags != nullptr;
+  }
+  if (tiled) {
     a.Kp = Kp;
-    const size_t xs = (size_t)Mp * Kp, ws = (size_t)Np * Kp;
-    int8_t* x8 = static_cast<int8_t*>(ds.i8_x.ensure(kI8Digits * xs, false));
-    int8_t* w8 = static_cast<int8_t*>(ds.i8_w.ensure(kI8Digits * ws, false));
-    // One digit count per 64x64 tile of the padded X and W (rewritten by every call).
-    const size_t fx = (size_t)(Mp / 64) * (Kp / 64), fw = (size_t)(Np / 64) * (Kp / 64);
-    uint8_t* flags = static_cast<uint8_t*>(ds.i8_flags.ensure(fx + fw, false));
     NarrowI8Args n{};
     n.X = a.X;
     n.W = a.W;
@@ -646,8 +614,8 @@ bool pipelined_host_layer(DeviceState& ds, int dev, int dtype, const LayerOp& op
   // Every host-buffer call is synchronous, so no earlier work on these or the
   // legacy stream can still touch the staging buffers.
   const int64_t dldx = (K + 3) & ~int64_t(3), dldy = (N + 3) & ~int64_t(3);
-  char* dx = static_cast<char*>(ds.stage[0].ensure((size_t)M * dldx * es, false));
-  char* dy = static_cast<char*>(ds.stage[3].ensure((size_t)M * dldy * es, false));
+  char* dx = static_cast<char*>(ds.stage[0].ensure((size_t)M * dldx * es));
+  char* dy = static_cast<char*>(ds.stage[3].ensure((size_t)M * dldy * es));
   DenseLaunch L{};
   L.dtype = dtype;
   L.epi = op.epi;
@@ -659,7 +627,7 @@ bool pipelined_host_layer(DeviceState& ds, int dev, int dtype, const LayerOp& op
     L.ldw = W.ld;
   } else {
     const int64_t dldw = (N + 3) & ~int64_t(3);
-    void* dw = ds.stage[1].ensure((size_t)K * dldw * es, false);
+    void* dw = ds.stage[1].ensure((size_t)K * dldw * es);
     stage_h2d(dw, dldw, W.base, W.ld, K, N, es, ds.pipe_up);
     L.w = dw;
     L.ldw = dldw;
@@ -668,7 +636,7 @@ bool pipelined_host_layer(DeviceState& ds, int dev, int dtype, const LayerOp& op
     if (is_device_pointer(op.b->base, dev)) {
       L.bias = op.b->base;
     } else {
-      void* d = ds.stage[2].ensure((size_t)N * es, false);
+      void* d = ds.stage[2].ensure((size_t)N * es);
       check_hip(hipMemcpyAsync(d, op.b->base, (size_t)N * es, hipMemcpyHostToDevice, ds.pipe_up),
                 "hipMemcpyAsync H2D");
       L.bias = d;
@@ -776,7 +744,7 @@ void sync_dense_chain(int dtype, const LayerOp* layers, int n, const Mat& Y) {
       return m.base;
     }
     const int64_t dld = (m.cols + 3) & ~int64_t(3);
-    void* d = buf.ensure((size_t)m.rows * dld * es, false);
+    void* d = buf.ensure((size_t)m.rows * dld * es);
     copy_h2d(d, dld, m, es, stream);
     *ld = dld;
     return d;
@@ -788,14 +756,14 @@ void sync_dense_chain(int dtype, const LayerOp* layers, int n, const Mat& Y) {
   for (int i = 0; i + 1 < n; ++i) inter = std::max(inter, M * ((layers[i].W->cols + 3) & ~int64_t(3)));
   void* hbuf[2] = {nullptr, nullptr};
   if (n > 1) {
-    hbuf[0] = ds.chain[0].ensure((size_t)inter * es, false);
-    if (n > 2) hbuf[1] = ds.chain[1].ensure((size_t)inter * es, false);
+    hbuf[0] = ds.chain[0].ensure((size_t)inter * es);
+    if (n > 2) hbuf[1] = ds.chain[1].ensure((size_t)inter * es);
   }
   const bool y_dev = is_device_pointer(Y.base, dev);
   const int64_t N_last = Y.cols;
   void* ystage = nullptr;
   int64_t ystage_ld = (N_last + 3) & ~int64_t(3);
-  if (!y_dev) ystage = ds.stage[3].ensure((size_t)M * ystage_ld * es, false);
+  if (!y_dev) ystage = ds.stage[3].ensure((size_t)M * ystage_ld * es);
 
   std::string plans;
   const void* prev = nullptr;
@@ -820,7 +788,7 @@ void sync_dense_chain(int dtype, const LayerOp* layers, int n, const Mat& Y) {
       if (is_device_pointer(op.b->base, dev)) {
         L.bias = op.b->base;
       } else {
-        void* d = ds.stage[2].ensure((size_t)L.N * es, false);
+        void* d = ds.stage[2].ensure((size_t)L.N * es);
         check_hip(hipMemcpyAsync(d, op.b->base, (size_t)L.N * es, hipMemcpyHostToDevice, stream),
                   "hipMemcpyAsync H2D");
         L.bias = d;
