@@ -14,6 +14,7 @@ import os
 import shutil
 import subprocess
 import sys
+import warnings
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG_DIR)  # ml-edsl_amd/
@@ -63,7 +64,7 @@ def build(jobs: int = 4, verbose: bool = False) -> str:
     os.replace(tmp, LIB_PATH)
     exts = [build_launch_module()]
     if importlib.util.find_spec("torch") is not None:  # the device API needs torch, the host API does not
-        exts.append(build_torch_launch_module())
+        exts += build_optional_torch_launch_module()
     if verbose:
         for path in [LIB_PATH, *exts]:
             print(f"built {path}")
@@ -91,9 +92,28 @@ def build_torch_launch_module() -> str:
         os.path.join(CSRC, "torch_launch.cpp"), f"-L{libs}", "-ltorch_python", "-ltorch_cpu", "-lc10"])
 
 
+def build_optional_torch_launch_module() -> list[str]:
+    """[its path]; [] with a warning where torch's headers or a C++ compiler are
+    not usable: the device API then checks operands in Python, as it does
+    without the module. No module of an earlier build is left behind."""
+    out = _module_path("_torch_launch")
+    try:
+        return [build_torch_launch_module()]
+    except (ImportError, OSError, RuntimeError) as e:
+        if os.path.exists(out):
+            os.remove(out)
+        warnings.warn(f"device launches check their operands in Python: {e}", stacklevel=2)
+        return []
+
+
+def _module_path(name: str) -> str:
+    import sysconfig
+    return os.path.join(PKG_DIR, name + sysconfig.get_config_var("EXT_SUFFIX"))
+
+
 def _link_module(name: str, cmd: list[str]) -> str:
     import sysconfig
-    out = os.path.join(PKG_DIR, name + sysconfig.get_config_var("EXT_SUFFIX"))
+    out = _module_path(name)
     tmp = out + ".tmp"
     cmd = [*cmd, "-fPIC", "-shared", "-Wall", f"-I{sysconfig.get_paths()['include']}", "-o", tmp, f"-L{PKG_DIR}",
            "-l:" + LIB_NAME, "-Wl,-rpath,$ORIGIN"]
