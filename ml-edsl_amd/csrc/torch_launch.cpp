@@ -108,4 +108,13 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_torch_launch", "Device launches o
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__torch_launch(void) { return PyModule_Create(&module); }
+// torch_build names the torch it was compiled against (build.torch_build_id);
+// the package uses it with no other.
+PyMODINIT_FUNC PyInit__torch_launch(void) {
+  PyObject* m = PyModule_Create(&module);
+  if (m != nullptr && PyModule_AddStringConstant(m, "torch_build", EDSL_TORCH_BUILD_ID) != 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -79,6 +79,12 @@ def build_launch_module() -> str:
     return _link_module("_launch", [cc, "-O2", os.path.join(CSRC, "pylaunch.c")])
 
 
+def torch_build_id(torch) -> str:
+    """The torch that a native module reads tensors of: their layout is that of
+    one build."""
+    return f"{torch.__version__} {torch.version.git_version}"
+
+
 def build_torch_launch_module() -> str:
     """Its counterpart on torch tensors (csrc/torch_launch.cpp), linked against
     torch's libraries, which the process has loaded before it imports this."""
@@ -88,7 +94,8 @@ def build_torch_launch_module() -> str:
     libs = os.path.join(os.path.dirname(torch.__file__), "lib")
     abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
     return _link_module("_torch_launch", [
-        cxx, "-O2", "-std=c++17", f"-D_GLIBCXX_USE_CXX11_ABI={abi}", *[f"-isystem{p}" for p in include_paths()],
+        cxx, "-O2", "-std=c++17", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
+        f'-DEDSL_TORCH_BUILD_ID="{torch_build_id(torch)}"', *[f"-isystem{p}" for p in include_paths()],
         os.path.join(CSRC, "torch_launch.cpp"), f"-L{libs}", "-ltorch_python", "-ltorch_cpu", "-lc10"])
 
 

@@ -9,11 +9,25 @@ library's.
 from __future__ import annotations
 
 from . import _native
+from .build import torch_build_id
 
 _native_launch = None  # checks and launch on torch tensors (csrc/torch_launch.cpp), once loaded
 _launch = None  # METH_FASTCALL binding of the two entries (csrc/pylaunch.c), once loaded
 _torch = None
 _raw_stream = None  # (current device index) -> raw hipStream_t of that device's current stream
+
+
+def _native_checks(torch):
+    """dense_launch of csrc/torch_launch.cpp, or None where the module is not
+    built or was built against another torch, whose tensors are laid out
+    otherwise (the checks below then run in Python)."""
+    try:
+        from . import _torch_launch
+    except ImportError:
+        return None
+    if getattr(_torch_launch, "torch_build", None) != torch_build_id(torch):
+        return None
+    return _torch_launch.dense_launch
 
 
 def _torch_module():
@@ -32,11 +46,7 @@ def _torch_module():
             _launch = fast
         except ImportError:
             _launch = None
-        try:
-            from ._torch_launch import dense_launch as native_launch
-            _native_launch = native_launch
-        except ImportError:
-            _native_launch = None
+        _native_launch = _native_checks(torch)
         get_dev = getattr(torch._C, "_cuda_getDevice", None)
         get_raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
         if get_dev is not None and get_raw is not None:
