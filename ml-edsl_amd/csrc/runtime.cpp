@@ -259,8 +259,10 @@ void check_dims(int64_t M, int64_t N, int64_t K) {
 }
 
 // Bytes of the partial tiles of a small-M plan with `ks` splits. The automatic
-// plans keep them within the scratch of the allocation-free launch, which takes
-// the same plans.
+// plans choose no split whose partials exceed the scratch of the allocation-free
+// launch, which takes the same plans; but a K tail makes one split two, and that
+// launch refuses the layer where two do not fit (M = 64: K % 16 != 0 and N >
+// 32768, W unaligned from K = 2048, aligned from 4096 or 2 N).
 constexpr size_t kGemvFixedScratch = EDSL_NOALLOC_SCRATCH_BYTES;
 size_t gemv_partials(int ks, int64_t M, int64_t N) {
   return (size_t)ks * 16 * ((M + 15) / 16) * ((N + 3) & ~int64_t(3)) * sizeof(float);

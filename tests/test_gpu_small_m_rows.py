@@ -64,3 +64,28 @@ def test_automatic_splits_fit_the_fixed_scratch(M, K, N):
     torch.cuda.synchronize()
     assert torch.equal(Y, Z)
     assert torch.allclose(Y, torch.addmm(b, X, W), rtol=0, atol=1e-4 * K ** 0.5)
+
+
+# A K tail needs two splits, whose partials do not fit from N = 32769 at M = 64
+# on: the allocation-free launch refuses such a layer where the small-M kernel
+# has it, and takes it where a tile does.
+@pytest.mark.parametrize("M, K, N, fits", [(64, 2049, 40001, False), (64, 4104, 40000, False), (64, 2049, 32765, True),
+                                           (64, 2047, 40001, True), (64, 4088, 40000, True)])
+def test_k_tails_and_the_fixed_scratch(M, K, N, fits):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(N)
+    X = torch.randn(M, K, device="cuda", generator=g)
+    W = torch.randn(K, N, device="cuda", generator=g)
+    Y = torch.zeros(M, N, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    args = (X.data_ptr(), K, W.data_ptr(), N, None, Y.data_ptr(), N, M, N, K, _native.EPI_NONE, 0.0, stream)
+    rc = _native.lib().edsl_hip_dense_f32_launch_noalloc(*args)
+    torch.cuda.synchronize()
+    if fits:
+        assert rc == 0, _native.last_error()
+    else:
+        assert rc == -5 and f"needs {512 * (N + 3 & ~3)} bytes" in str(_native.last_error()), _native.last_error()
+        assert not Y.any()
+        assert _native.lib().edsl_hip_dense_f32_launch(*args) == 0, _native.last_error()
+        torch.cuda.synchronize()
+    assert torch.allclose(Y, X @ W, rtol=0, atol=1e-4 * K ** 0.5)
