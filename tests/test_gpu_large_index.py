@@ -1,9 +1,9 @@
 """Outputs beyond 2^31 elements: every kernel family indexes with 64-bit
 offsets where a 32-bit product would overflow. Each case builds device
-operands directly (8 GiB outputs, or 8 GiB weights for the small-M
-streaming kernel), runs one launch through the C ABI,
-and checks sampled rows / columns -- always including the last ones, where
-the offsets are largest -- against the oracle on the same slices.
+operands directly (8 GiB outputs, 8 GiB weights for the small-M streaming
+kernel, 8 GiB of digit planes), runs one launch through the C ABI, and checks
+sampled rows / columns -- always including the last ones, where the offsets are
+largest -- against the oracle on the same slices.
 """
 from __future__ import annotations
 
@@ -45,6 +45,73 @@ def test_tiled_f32_output_beyond_2_31(torch_cuda):
     ref = oracle.dense_f32_chains(X.index_select(0, rows).cpu().numpy(), W.cpu().numpy(), b.cpu().numpy(), "relu")
     assert_f32_parity(Y.index_select(0, rows).cpu().numpy(), ref, K)
     del X, W, b, Y
+    torch.cuda.empty_cache()
+
+
+def test_split_f32_output_beyond_2_31(torch_cuda):
+    """The bf16 matrix cores at fp32 precision: C's descriptors, from a tile's
+    first row, are cut at 2^31 - 1 bytes, where masked columns are sent."""
+    torch = torch_cuda
+    from mlir_edsl_hip.device import dense_launch
+    M, K, N = 65535, 256, 32768 + 257  # Y: 2.16e9 elements; partial tiles at both edges
+    g = torch.Generator(device="cuda").manual_seed(8)
+    X = torch.randn(M, K, device="cuda", generator=g)
+    W = torch.randn(K, N, device="cuda", generator=g)
+    b = torch.randn(N, device="cuda", generator=g)
+    buf = torch.full((M * N + 4096,), 7.0, device="cuda")
+    Y = buf[:M * N].view(M, N)
+    dense_launch(X, W, b, Y, _native.EPI_BIAS_RELU)
+    torch.cuda.synchronize()
+    plan = _native.last_plan()
+    assert plan.startswith("gemm_f32 split=bf16x6 "), plan
+    rows = _rows(torch, M)
+    ref = oracle.dense_f32_chains(X.index_select(0, rows).cpu().numpy(), W.cpu().numpy(), b.cpu().numpy(), "relu")
+    assert_f32_parity(Y.index_select(0, rows).cpu().numpy(), ref, K)
+    assert bool((buf[M * N:] == 7.0).all())
+    del X, W, b, Y, buf
+    torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("M, K, N, tile", [(255, 1024, 32767, "256x128x16"), (256, 4096, 16383, "128x128x32_w8")])
+def test_split_f32_rows_at_the_largest_stride(M, K, N, tile, torch_cuda):
+    """A row stride of 2^21 - 1, the largest the split tiles take: the last rows
+    of a 256-row tile lie just under 2^31 bytes from its first."""
+    torch = torch_cuda
+    from mlir_edsl_hip.device import dense_launch
+    ldc = 2**21 - 1
+    g = torch.Generator(device="cuda").manual_seed(N)
+    X = torch.randn(M, K, device="cuda", generator=g)
+    W = torch.randn(K, N, device="cuda", generator=g)
+    buf = torch.full((M, ldc), 7.0, device="cuda")
+    dense_launch(X, W, None, buf[:, :N], _native.EPI_NONE)
+    torch.cuda.synchronize()
+    plan = _native.last_plan()
+    assert plan.startswith(f"gemm_f32 split=bf16x6 tile={tile} "), plan
+    rows = _rows(torch, M)
+    ref = oracle.dense_f32_chains(X.index_select(0, rows).cpu().numpy(), W.cpu().numpy(), None, "none")
+    assert_f32_parity(buf[:, :N].index_select(0, rows).cpu().numpy(), ref, K)
+    assert bool((buf[:, N:] == 7.0).all())  # nothing else was written
+    del X, W, buf
+    torch.cuda.empty_cache()
+
+
+def test_digit_planes_beyond_2_31(torch_cuda):
+    """Values of all four digits with planes of 2^31 bytes each."""
+    torch = torch_cuda
+    from mlir_edsl_hip.device import dense_launch
+    M, K, N = 131072, 16384, 128
+    g = torch.Generator(device="cuda").manual_seed(9)
+    X = torch.randint(-2**31, 2**31 - 1, (M, K), device="cuda", dtype=torch.int32, generator=g)
+    W = torch.randint(-2**31, 2**31 - 1, (K, N), device="cuda", dtype=torch.int32, generator=g)
+    Y = torch.empty(M, N, device="cuda", dtype=torch.int32)
+    dense_launch(X, W, None, Y, _native.EPI_NONE)
+    torch.cuda.synchronize()
+    plan = _native.last_plan()
+    assert plan.startswith("narrow_i8+gemm_i8 variant="), plan
+    rows = _rows(torch, M)
+    ref = oracle.dense_i32(X.index_select(0, rows).cpu().numpy(), W.cpu().numpy(), None, "none")
+    assert np.array_equal(Y.index_select(0, rows).cpu().numpy(), ref)
+    del X, W, Y
     torch.cuda.empty_cache()
 
 
