@@ -18,10 +18,10 @@
 // The products left out, ml, lm and ll, are below 2^-24 of a product together.
 // An fp32 chain of n terms is within n 2^-24 sum |ab| of the exact sum and this
 // one within 2 2^-24 of it, so only an output of a single term can lose by the
-// omission. Such an output has a row of A or a column of B with at most one
-// nonzero value. A workgroup therefore counts the nonzero values of its rows and
-// columns in the first three steps and, where one has fewer than two, takes
-// eight products (all but ll, below 2^-33).
+// omission. A workgroup therefore counts the nonzero values of its rows and
+// columns in its first 48 or 64 k and, unless the emptiest row and the emptiest
+// column must meet at two k there (together two more nonzero values than there
+// are k), takes eight products (all but ll, below 2^-33).
 //
 // Relative 2-norm error against float64, this kernel / the fp32 MFMA chain:
 // N(0,1) data at K = 1024, 2048, 4096 1.9e-7 / 5.7e-7, 2.7e-7 / 8.1e-7, 4.0e-7
@@ -216,7 +216,9 @@ gemm_f32_split_kernel(GemmF32Args args) {
   constexpr int RB = C::RB, CB = C::CB, KK = C::KK;
   __shared__ __align__(16) char smem[C::kLds];
   __shared__ int counts[C::BM + C::BN];  // nonzero values of the tile's rows and columns in the first steps
+  __shared__ int fewest[2];              // of a row, of a column
   __shared__ int biggest;
+  if (threadIdx.x < 2) fewest[threadIdx.x] = 1 << 30;
   for (int i = threadIdx.x; i < C::BM + C::BN; i += C::kThreads) counts[i] = 0;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -327,9 +329,21 @@ gemm_f32_split_kernel(GemmF32Args args) {
     atomicAdd(&counts[line_of(o)], n);
   }
   __syncthreads();
+  for (int i = threadIdx.x; i < C::BM + C::BN; i += C::kThreads) {  // whole waves, of rows or of columns
+    int n = counts[i];
+    n = min(n, __builtin_amdgcn_update_dpp(n, n, 0x121, 0xf, 0xf, false));  // of 16 lanes, by rotation
+    n = min(n, __builtin_amdgcn_update_dpp(n, n, 0x122, 0xf, 0xf, false));
+    n = min(n, __builtin_amdgcn_update_dpp(n, n, 0x124, 0xf, 0xf, false));
+    n = min(n, __builtin_amdgcn_update_dpp(n, n, 0x128, 0xf, 0xf, false));
+    if (lane % 16 == 0) atomicMin(&fewest[i >= C::BM], n);
+  }
+  __syncthreads();
   bool sparse = full < kCheck;  // its last step has been counted more than once
-  for (int i = threadIdx.x; i < C::BM + C::BN; i += C::kThreads) sparse |= counts[i] < 2;
-  const bool eight = __syncthreads_or(sparse) != 0;  // uniform: take ml and lm
+  sparse |= fewest[0] + fewest[1] < kCheck * C::BK + 2;
+  // Uniform: take ml and lm. (A vote although all threads agree: with the flag read
+  // back by readfirstlane the compiler spills registers in the loop of six
+  // products, 10000x500x1000 86 us against 74.)
+  const bool eight = __syncthreads_or(sparse) != 0;
 
   constexpr int BS = KK == 1 ? 2 : KK;  // sets of B fragments
   bf16x8 a[2][kPlanes], b[BS][CB][kPlanes];

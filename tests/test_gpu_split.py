@@ -85,8 +85,10 @@ def test_split_epilogues(epi, has_bias, act):
 
 
 # Operands with few terms a sum, where fp32 rounds once a term: one nonzero value
-# a row or a column, n of them in different steps, and half of all zero.
-@pytest.mark.parametrize("what", ["one_a_row", "one_a_column", "two_a_row", "eight_a_row", "thirty_a_row", "relu"])
+# a row or a column, n of them in different steps, rows of two and full columns
+# that meet at one k, and half of all zero on one or both sides.
+@pytest.mark.parametrize("what", ["one_a_row", "one_a_column", "two_a_row", "eight_a_row", "thirty_a_row",
+                                  "one_in_common", "relu", "relu_both"])
 @pytest.mark.parametrize("M, K, N", [(2500, 1030, 2496), (2001, 543, 2003), (4000, 271, 4001)],
                          ids=["256x128", "128x128_w8", "128x128"])
 def test_sparse_operands_lose_no_precision(M, K, N, what):
@@ -100,8 +102,13 @@ def test_sparse_operands_lose_no_precision(M, K, N, what):
         d = torch.zeros_like(W)
         d[c % K, c] = W[0]
         W = d
-    elif what == "relu":
+    elif what.startswith("relu"):
         X.relu_()
+        if what == "relu_both":
+            W.relu_()
+    elif what == "one_in_common":
+        X[:, 2:] = 0.0
+        W[1] = 0.0
     else:
         d = torch.zeros_like(X)
         n = {"one_a_row": 1, "two_a_row": 2, "eight_a_row": 8, "thirty_a_row": 30}[what]
