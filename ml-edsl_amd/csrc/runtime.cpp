@@ -272,8 +272,12 @@ size_t gemv_partials(int ks, int64_t M, int64_t N) {
 // workgroup. For each, the K split is the one of least cost: the time of the
 // rounds of workgroups over the CUs, in units of a full chip, plus the bytes
 // of the partial sums (written and read once) over those of W. The first width
-// that keeps three quarters of the CUs busy is taken; when none does, the plan
-// with the most workgroups. Every wave keeps >= 2 steps of 16 rows. The order
+// that keeps three quarters of the CUs busy is taken, or, where W is below 16
+// MiB and its rows start on 128-byte lines, a later one that gives every CU a
+// workgroup with K in at least as many slices (13x2036x896 9.0 us on 64 columns x
+// 15 splits, 7.6 on 32 x 8; with rows off the lines narrow blocks share them:
+// 2x1424x2076 6.7 us on 128 columns, 7.3 on 32); when none does, the plan with
+// the most workgroups. Every wave keeps >= 2 steps of 16 rows. The order
 // is measured (M=16, K=N=8192 on MI355X): 128 columns x 4 splits beat 256 x 8
 // (more partial traffic), 64 x 2 (256-byte row runs) and 32 x 1 (8-byte loads:
 // the per-CU request rate, not the byte count, limits a streaming workgroup).
@@ -281,15 +285,18 @@ size_t gemv_partials(int ks, int64_t M, int64_t N) {
 // splits put two workgroups on 8 of the CUs (40.3 us against 28.0 us for 7). A
 // forced split (edsl_hip_set_gemv_ksplit) limits the choice to the widths that
 // can take it.
-bool plan_gemv(const DeviceState& ds, int64_t M, int64_t N, int64_t K, int* cols_out, int* ks_out) {
+bool plan_gemv(const DeviceState& ds, int64_t M, int64_t N, int64_t K, int w_mode, int* cols_out,
+               int* ks_out, bool* narrowed_out) {
   static const int kCols[] = {128, 256, 64, 32};
   if (N < 1 || K % 16 != 0) return false;
   int best_cols = 0, best_ks = 0;
-  int64_t best_wgs = 0;
+  int64_t best_wgs = 0, best_slices = 0;
+  *narrowed_out = false;
   // K is walked in 16-row chunks spread evenly over the ks x wk wave slices;
   // the automatic plan gives every slice at least two, a forced split at
   // least one.
   const int64_t chunks = K / 16;
+  const bool may_narrow = w_mode == kWVector && K * N * (int64_t)sizeof(float) < 16 << 20;
   // Returns true when the width fills the chip.
   auto consider = [&](int cols) {
     if (g_force_cols > 0 && cols != g_force_cols) return false;
@@ -297,6 +304,7 @@ bool plan_gemv(const DeviceState& ds, int64_t M, int64_t N, int64_t K, int* cols
     // The last column block may be partial (its lanes past N read the last
     // columns and store nothing).
     const int64_t groups = (N + cols - 1) / cols;
+    const bool narrow = 4 * best_wgs >= 3 * ds.cus && g_force_ksplit == 0;
     int ks = 1;
     if (g_force_ksplit > 0) {
       // A forced split is taken only by widths that can honour it.
@@ -305,24 +313,31 @@ bool plan_gemv(const DeviceState& ds, int64_t M, int64_t N, int64_t K, int* cols
     } else {
       if (chunks < 2 * wk) return false;
       double best = 0;
-      for (int s = 1; s <= gemv_f32_max_ksplit() && chunks >= 2 * wk * s; ++s) {
+      int least = 1;
+      if (narrow) least = (int)((best_slices + wk - 1) / wk);
+      if (narrow && (least > gemv_f32_max_ksplit() || chunks < 2 * wk * least ||
+                     gemv_partials(least, M, N) > kGemvFixedScratch))
+        return false;
+      for (int s = least; s <= gemv_f32_max_ksplit() && chunks >= 2 * wk * s; ++s) {
         if (s > 1 && gemv_partials(s, M, N) > kGemvFixedScratch) break;
         const int64_t rounds = (groups * s + ds.cus - 1) / ds.cus;
         const double cost = (double)(rounds * ds.cus) / (double)(groups * s) +
                             (s > 1 ? 2.0 * (double)s * (double)M / (double)K : 0.0);
-        if (s == 1 || cost < best) {
+        if (s == least || cost < best) {
           best = cost;
           ks = s;
         }
       }
     }
     const int64_t wgs = groups * ks;
-    if (wgs > best_wgs) {
+    if (narrow ? wgs >= ds.cus : wgs > best_wgs) {
       best_cols = cols;
       best_ks = ks;
       best_wgs = wgs;
+      best_slices = ks * wk;
+      *narrowed_out = narrow;
     }
-    return 4 * wgs >= 3 * ds.cus;
+    return best_wgs >= ds.cus || (4 * best_wgs >= 3 * ds.cus && (!may_narrow || g_force_ksplit > 0));
   };
   for (int cols : kCols)
     if (consider(cols)) break;
@@ -344,6 +359,7 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
   // Small M: the streaming kernel walks the first K16 = K - K % 16 rows; the
   // reduce kernel adds the rest. Operands need no alignment.
   int gemv_cols = 0, gemv_ks = 0;
+  bool gemv_narrowed = false;
   const bool w_vec = al16(L.w) && al16(L.y) && (!bias_al || al16(bias_al)) && L.ldw % 4 == 0 &&
                      L.ldy % 4 == 0 && N % 4 == 0;
   const int K16 = K & ~15;
@@ -402,7 +418,9 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
   }
 
   small_m = small_m || g_force_ksplit > 0 || g_force_small_m == 1;
-  if (small_m && M >= 1 && M <= kGemvMaxM && K16 > 0 && plan_gemv(ds, M, N, K16, &gemv_cols, &gemv_ks)) {
+  const int w_mode = gemv_f32_w_mode(static_cast<const float*>(L.w), L.ldw, N);
+  if (small_m && M >= 1 && M <= kGemvMaxM && K16 > 0 &&
+      plan_gemv(ds, M, N, K16, w_mode, &gemv_cols, &gemv_ks, &gemv_narrowed)) {
     const bool tail = K16 < K;
     if (tail && gemv_ks == 1) gemv_ks = 2;  // the reduce kernel adds the tail
     GemvF32Args a{};
@@ -426,7 +444,7 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
     const bool scratch = a.ksplit > 1;
     const size_t part_bytes = scratch ? gemv_partials(a.ksplit, M, N) : 0;
     if (!has_bias) a.bias = nullptr;
-    a.w_mode = gemv_f32_w_mode(a.W, a.ldw, N);
+    a.w_mode = w_mode;
     // A split below the power of two that gives every CU a workgroup leaves
     // longer chains, which a second set of accumulators shortens again
     // (unaligned rows from 3/4 of it down: 48x4096x4097 on 7 of 8, 1.6e-7
@@ -434,7 +452,7 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
     // of all of K: 48x4096x50257 4.1e-7 with one set).
     int full = w_vec ? 1 : 2;
     while (full < gemv_f32_max_ksplit() && ((int64_t)N + gemv_cols - 1) / gemv_cols * full < ds.cus) full *= 2;
-    a.two_sets = w_vec ? a.ksplit < full : 4 * a.ksplit < 3 * full;
+    a.two_sets = gemv_narrowed || (w_vec ? a.ksplit < full : 4 * a.ksplit < 3 * full);
     if (fixed) {
       // Caller-fixed scratch: nothing is allocated and no cross-stream
       // ordering is added.
