@@ -392,8 +392,6 @@ int plan_f32_small(const F32TileQuery& q, bool stream_rows) {
       if (2 * tiles > 5 * q.cus) return 0;
     } else if (gemm_f32_config(cfg).guard == kGuardScalar) {
       if (2 * tiles > 9 * q.cus) return 0;
-      const int64_t t32 = ((q.M + 31) / 32) * ((q.N + 31) / 32);
-      if (2 * tiles > 5 * q.cus && q.K > 320 && q.ldb % 2 == 0 && t32 <= q.cus) return 0;
     } else {
       return 0;
     }

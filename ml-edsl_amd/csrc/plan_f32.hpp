@@ -93,10 +93,9 @@ int plan_f32_tile(const F32TileQuery& q);
 //    9.4 / 5.0, 300x512x300 6.9 / 5.0, 400x256x400 4.9 / 4.4; with more
 //    they tie or lose (100x64x2000 4.0 / 4.1, 512x64x512 3.7 / 4.2);
 //  * the any-shape tiles, up to 4.5: 255x255x255 7.3 / 3.3, 401x511x399
-//    10.6 / 7.1, 513x1023x511 20.4 / 16.4; up to 2.5 from K = 321 on where W's
-//    rows are 8-byte aligned and 32x32 tiles fit one round, which they then do
-//    faster (32x323x7146 8.7 / 10.9, 128x646x1728 with rows of 1732 9.7 / 12.1,
-//    138x450x1280 with rows of 1284 8.0 / 8.7; but 64x515x2674 9.8 / 8.6);
+//    10.6 / 7.1, 513x1023x511 20.4 / 16.4. (Where W's rows are 8-byte aligned and
+//    32x32 tiles fit one round those may be faster, 32x323x7146 8.7 / 10.9, 385x505x456
+//    10.2 / 8.7, but their sums are in longer chains: 2.0e-7 from float64 / 1.0e-7);
 //  * the other tiles (32x32 R x C and larger) fill the chip and win:
 //    512x256x512 3.9 / 5.7; the exact 16x16 tile too: 128x128x128 2.4 / 2.5.
 // Eight waves from K = 449 on (16x512x4096 3.9 with four, 3.7 with eight;
