@@ -447,12 +447,16 @@ void launch_f32(DeviceState& ds, const DenseLaunch& L, hipStream_t stream, const
     a.w_mode = w_mode;
     // A split below the power of two that gives every CU a workgroup leaves
     // longer chains, which a second set of accumulators shortens again
-    // (unaligned rows from 3/4 of it down: 48x4096x4097 on 7 of 8, 1.6e-7
-    // against float64 either way, is 4 % faster with one; one split has chains
-    // of all of K: 48x4096x50257 4.1e-7 with one set).
+    // (unaligned rows below 7/8 of it: 48x4096x4097 on 7 of 8, 1.6e-7 against
+    // float64 either way, is 4 % faster with one; one split has chains of all of
+    // K: 48x4096x50257 4.1e-7 with one set). So does a width that all 16 splits
+    // do not give every CU a workgroup, where narrower ones would have had more
+    // slices (37x4232x1760 1.85e-7 with one set, 1.59e-7 on 64 columns).
+    const int64_t groups = ((int64_t)N + gemv_cols - 1) / gemv_cols;
     int full = w_vec ? 1 : 2;
-    while (full < gemv_f32_max_ksplit() && ((int64_t)N + gemv_cols - 1) / gemv_cols * full < ds.cus) full *= 2;
-    a.two_sets = gemv_narrowed || (w_vec ? a.ksplit < full : 4 * a.ksplit < 3 * full);
+    while (full < gemv_f32_max_ksplit() && groups * full < ds.cus) full *= 2;
+    a.two_sets = gemv_narrowed || groups * full < ds.cus ||
+                 (w_vec ? a.ksplit < full : 8 * a.ksplit < 7 * full);
     if (fixed) {
       // Caller-fixed scratch: nothing is allocated and no cross-stream
       // ordering is added.

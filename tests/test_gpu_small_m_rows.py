@@ -66,6 +66,23 @@ def test_automatic_splits_fit_the_fixed_scratch(M, K, N):
     assert torch.allclose(Y, torch.addmm(b, X, W), rtol=0, atol=1e-4 * K ** 0.5)
 
 
+# Three and four row blocks on plans with fewer slices of K than the workgroups of
+# powers of two had: one set of accumulators was 1.85e-7, 2.04e-7 and 1.54e-7 from
+# float64 there, slices as many as before 1.59e-7, 1.77e-7 and 1.47e-7.
+@pytest.mark.parametrize("M, K, N, bound", [(37, 4232, 1760, 1.65e-7), (39, 4735, 1596, 1.85e-7), (42, 2529, 1295, 1.5e-7)])
+def test_fewer_slices_keep_their_precision(M, K, N, bound):
+    import torch
+    from mlir_edsl_hip.device import dense_launch
+    g = torch.Generator(device="cuda").manual_seed(K)
+    X = torch.randn(M, K, device="cuda", generator=g)
+    W = torch.randn(K, N, device="cuda", generator=g)
+    Y = torch.empty(M, N, device="cuda")
+    dense_launch(X, W, None, Y, _native.EPI_NONE)
+    exact = X.double() @ W.double()
+    assert _native.last_plan().startswith("gemv_f32 mb=3 "), _native.last_plan()
+    assert ((Y.double() - exact).norm() / exact.norm()).item() <= bound
+
+
 # A K tail needs two splits, whose partials do not fit from N = 32769 at M = 64
 # on: the allocation-free launch refuses such a layer where the small-M kernel
 # has it, and takes it where a tile does.
