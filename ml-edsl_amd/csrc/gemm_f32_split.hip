@@ -67,8 +67,8 @@
 // register-only loop of the same MFMAs takes 491 us at 4096^3. The 256x128 tile
 // of four waves, each 128x64, reads LDS least of the tiles whose two sets of
 // accumulators fit the registers (a 256x256 tile with one took 580 us at the
-// error above). Measured, us, against the fp32 tiles: 4096^3 650-662 / 905
-// (208-211 TFLOP/s; 700 / 905 on eight products), 4000x1024x4000 178 / 245,
+// error above). Measured, us, against the fp32 tiles: 4096^3 650-691 / 905
+// by box (199-211 TFLOP/s; 700 / 905 on eight products), 4000x1024x4000 178 / 245,
 // 2500^3 184 / 277; 2048^3 on eight waves of 64x32 97 / 120, 2001^3 99 / 159;
 // 10000x500x1000 on two workgroups of 128x128x16 per CU 75 / 94 (83 on eight
 // waves), 3333^3 428 / 681. Counting the first steps and testing the sums cost
