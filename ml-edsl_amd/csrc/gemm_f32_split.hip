@@ -503,20 +503,21 @@ gemm_f32_split_kernel(GemmF32Args args) {
     const int half = lane >> 5, l32 = lane & 31;
     const int ldc = (int)args.ldc;
     const i32x4 rsrc = buffer_rsrc(args.C + (int64_t)m0 * ldc, (int64_t)(M - m0) * ldc * 4);
+    const int col0 = n0 + wn * CB * 32 + l32;
+    float bv[CB];
 #pragma unroll
-    for (int j = 0; j < CB; ++j) {
-      const int col = n0 + (wn * CB + j) * 32 + l32;
-      const float bv = epi_has_bias(EPI) && col < N ? args.bias[col] : 0.0f;
+    for (int j = 0; j < CB; ++j) bv[j] = epi_has_bias(EPI) && col0 + 32 * j < N ? args.bias[col0 + 32 * j] : 0.0f;
 #pragma unroll
-      for (int i = 0; i < RB; ++i) {
-        const int at = (((wm * RB + i) * 32 + 4 * half) * ldc + col) * 4;
+    for (int i = 0; i < RB; ++i) {
+      const int at = (((wm * RB + i) * 32 + 4 * half) * ldc + col0) * 4;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int dr = 8 * (r >> 2) + (r & 3);
-          raw_buffer_store_f32(apply_epilogue_f32<EPI>(acc[i][j][r], bv, args.alpha), rsrc,
-                               col < N ? at + dr * ldc * 4 : 0x7fffffff, 0, kAuxNonTemporal);
-        }
-        __builtin_amdgcn_sched_barrier(0);
+      for (int r = 0; r < 16; ++r) {
+        const int dr = 8 * (r >> 2) + (r & 3);
+#pragma unroll
+        for (int j = 0; j < CB; ++j)
+          raw_buffer_store_f32(apply_epilogue_f32<EPI>(acc[i][j][r], bv[j], args.alpha), rsrc,
+                               col0 + 32 * j < N ? at + dr * ldc * 4 + 128 * j : 0x7fffffff, 0, kAuxNonTemporal);
+        if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
       }
     }
     return true;
