@@ -507,19 +507,27 @@ gemm_f32_split_kernel(GemmF32Args args) {
     float bv[CB];
 #pragma unroll
     for (int j = 0; j < CB; ++j) bv[j] = epi_has_bias(EPI) && col0 + 32 * j < N ? args.bias[col0 + 32 * j] : 0.0f;
+    auto store = [&](auto aux) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < RB; ++i) {
-      const int at = (((wm * RB + i) * 32 + 4 * half) * ldc + col0) * 4;
+      for (int i = 0; i < RB; ++i) {
+        const int at = (((wm * RB + i) * 32 + 4 * half) * ldc + col0) * 4;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int dr = 8 * (r >> 2) + (r & 3);
+        for (int r = 0; r < 16; ++r) {
+          const int dr = 8 * (r >> 2) + (r & 3);
 #pragma unroll
-        for (int j = 0; j < CB; ++j)
-          raw_buffer_store_f32(apply_epilogue_f32<EPI>(acc[i][j][r], bv[j], args.alpha), rsrc,
-                               col0 + 32 * j < N ? at + dr * ldc * 4 + 128 * j : 0x7fffffff, 0, kAuxNonTemporal);
-        if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+          for (int j = 0; j < CB; ++j)
+            raw_buffer_store_f32(apply_epilogue_f32<EPI>(acc[i][j][r], bv[j], args.alpha), rsrc,
+                                 col0 + 32 * j < N ? at + dr * ldc * 4 + 128 * j : 0x7fffffff, 0, decltype(aux)::value);
+          if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
       }
-    }
+    };
+    // Rows of C on 128-byte lines are streamed; lines that two segments share stay
+    // in the caches until both are there (3310x288x2369 40.4 -> 35.7 us).
+    if (ldc % 32 == 0 && reinterpret_cast<uintptr_t>(args.C) % 128 == 0)
+      store(std::integral_constant<int, kAuxNonTemporal>{});
+    else
+      store(std::integral_constant<int, 0>{});
     return true;
   };
   const bool done = eight ? compute(std::integral_constant<int, 8>{}) : compute(std::integral_constant<int, 6>{});
